@@ -162,24 +162,38 @@ __device__ __forceinline__ EdgeRec load_edge(cptr<EdgeRec> ec, int k) {
     return e;
 }
 
-// Crossing term of an edge that lies entirely right of the wave (flag
-// kCullFarCrossExact): +1 on the rows an upward edge spans, -1 for a
-// downward one; cross_term evaluates to the same value there.
-__device__ __forceinline__ void row_cross_term(const EdgeRec& E, float py, Geom& G) {
-    const bool b0 = E.y0 <= py, b1 = E.y1 <= py;
-    G.winding += (b0 != b1) ? (b0 ? 1 : -1) : 0;
-}
-
 // Edge classes of one 64-edge chunk starting at edge c (lane k: edge c + k,
-// cull words q), as ballots.  All exact:
+// cull words q), the first two as ballots.  All exact:
 //   dist   near (distance can matter): distance term, and the crossing term
 //          when the edge spans a row;
 //   cross  exact crossing terms: spans a row and is near or not flagged;
-//   right  far, spans a row, flagged, right of the wave: row-span crossing
-//          term only (far, flagged, left: nothing -- its crossing term is 0).
+//   right  far, spans a row, flagged, right of the wave: its crossing term is
+//          +1 (upward) or -1 on every row it spans, as cross_term evaluates
+//          it there (far, flagged, left: its crossing term is 0).
+// The right edges' terms are summed here for the wave's eight rows at once,
+// without their geometry: the rows an edge spans are in its cull words
+// (exact), so lane k makes its edge's terms as one byte per row (rows 0-3 in
+// right_lo, 4-7 in right_hi), and two DPP sums add the lanes.  A row's sum
+// lies in [-64, 64], so row_term reads it back without carries between rows.
+// The edge walk visited each of these edges with a scalar load instead; the
+// entries of a chain that is not closed bit for bit (every chain once an
+// optimizer has moved the segments' copies of a shared end point) took that
+// walk even where no edge is near.  Training step of 4096 drifted rings at
+// 2040 x 1356: forward 155.6 -> 138.3 us, backward 108.2 -> 99.9 us (fewer
+// records); 16384 clustered rings at 2048 x 2048: 210.8 -> 197.4 and
+// 119.8 -> 105.5 us.
 struct ChunkMasks {
-    uint64_t dist, cross, right;
+    uint64_t dist, cross;
+    int32_t right_lo, right_hi;
+    int nright;   // (counting instantiation)
 };
+
+// The summed right terms of the wave's row lane >> 4 (from right_lo; row
+// 4 + (lane >> 4) from right_hi).
+__device__ __forceinline__ int row_term(int32_t right) {
+    const uint32_t biased = (uint32_t)right + 0x80808080u;
+    return (int)((biased >> ((threadIdx.x & 0x30u) >> 1)) & 0xffu) - 128;
+}
 
 template <bool CROSS>
 __device__ __forceinline__ ChunkMasks chunk_masks(int4 q, int c, int e1, const WaveRect& W) {
@@ -189,12 +203,29 @@ __device__ __forceinline__ ChunkMasks chunk_masks(int4 q, int c, int e1, const W
     ChunkMasks m;
     m.dist = __ballot(dn);
     m.cross = 0ull;
-    m.right = 0ull;
+    m.right_lo = m.right_hi = 0;
+    m.nright = 0;
     if constexpr (CROSS) {
         const bool cb = in && span_hits(packed_lo(q.y), packed_span(q.y), W.r1);
         const bool flagged = (q.w & kCullFarCrossExact) != 0;
         m.cross = __ballot(cb && (dn || !flagged));
-        m.right = __ballot(cb && !dn && flagged && packed_lo(q.z) > W.c1);
+        const bool rt = cb && !dn && flagged && packed_lo(q.z) > W.c1;
+        const uint64_t mright = __ballot(rt);
+        if (mright) {
+            m.nright = __builtin_popcountll(mright);
+            // Rows a..b of the wave (0 <= a <= b <= 7 where rt holds).
+            const int lo = packed_lo(q.y) - W.r0;
+            const int a = max(lo, 0);
+            const int b = min(lo + packed_span(q.y) - kWaveRowsExt, kWaveRowsExt);
+            const uint64_t ones = 0x0101010101010101ull;
+            const uint64_t rows = (ones << ((8 * a) & 63)) & (ones >> ((8 * (kWaveRowsExt - b)) & 63));
+            const bool up = (q.w & kCullUp) != 0;
+            const uint32_t l = (uint32_t)rows, h = (uint32_t)(rows >> 32);
+            const uint32_t sl = wave_incl_scan_u32(rt ? (up ? l : 0u - l) : 0u);
+            const uint32_t sh = wave_incl_scan_u32(rt ? (up ? h : 0u - h) : 0u);
+            m.right_lo = __builtin_amdgcn_readlane((int)sl, kWave - 1);
+            m.right_hi = __builtin_amdgcn_readlane((int)sh, kWave - 1);
+        }
     }
     return m;
 }
@@ -207,11 +238,11 @@ __device__ __forceinline__ void chunk_geometry(const ChunkMasks& cm, int c,
                                                cptr<EdgeRec> edges, float px,
                                                const float (&py)[kPix], Geom (&G)[kPix],
                                                EvalCounts& n, int npix) {
-    const uint64_t mdn = cm.dist, mcross = cm.cross, mright = cm.right;
+    const uint64_t mdn = cm.dist, mcross = cm.cross;
     if constexpr (COUNT) {
         n.dist += (uint64_t)__builtin_popcountll(mdn) * npix;
         n.cross += (uint64_t)__builtin_popcountll(mcross) * npix;
-        n.row += (uint64_t)__builtin_popcountll(mright) * npix;
+        n.row += (uint64_t)cm.nright * npix;
     }
     const cptr<EdgeRec> ec = edges + c;
     if constexpr (BEST > 0) {
@@ -256,10 +287,10 @@ __device__ __forceinline__ void chunk_geometry(const ChunkMasks& cm, int c,
 #pragma unroll
             for (int p = 0; p < kPix; ++p) cross_term(E, wx, py[p] - E.y0, py[p], G[p]);
         }
-        for (uint64_t todo = mright; todo; todo &= todo - 1) {
-            const EdgeRec E = load_edge(ec, (int)__builtin_ctzll(todo));
-#pragma unroll
-            for (int p = 0; p < kPix; ++p) row_cross_term(E, py[p], G[p]);
+        if (cm.right_lo | cm.right_hi) {
+            static_assert(kPix == 2, "one pixel row per lane in each of the packed sums");
+            G[0].winding += row_term(cm.right_lo);
+            G[1].winding += row_term(cm.right_hi);
         }
     }
 }
@@ -460,50 +491,35 @@ __device__ __forceinline__ bool prim_culled_lane(const PrimRec* __restrict__ p,
     return !near & ((closed != 0) | !span_hits(a.z, a.w, W.r1) | (W.c0 > b.z));
 }
 
-// Winding number at the pixel row r of a wave over the edges c + lane < e1 of
-// one chunk, when none of them has a distance or exact crossing term for the
-// wave (a far chunk): an edge whose crossing rows (exact) contain r is then
-// flagged kCullFarCrossExact and misses the wave's near columns, so its
-// crossing term there is +1 (upward) or -1 when it lies right of the wave and
-// 0 when it lies left -- the values cross_term computes at every pixel of
-// that row.  One lane per edge, two ballots; no edge geometry is read.
-__device__ __forceinline__ int far_winding(int4 q, int c, int e1, const WaveRect& W) {
-    const bool in = c + (int)(threadIdx.x & (kWave - 1)) < e1;
-    const bool hit = in && span_hits(packed_lo(q.y), packed_span(q.y) - kWaveRowsExt, W.r0) &&
-                     packed_lo(q.z) > W.c1;
-    const bool up = (q.w & kCullUp) != 0;
-    return __builtin_popcountll(__ballot(hit && up)) - __builtin_popcountll(__ballot(hit && !up));
-}
-
 // Far entry: no edge of the primitive lies within the cull distance of any of
 // the wave's pixels (its near ranges miss the wave), and (fill) every edge
 // whose y-range spans one of the wave's rows carries kCullFarCrossExact.
-// Then no pixel needs the exact coverage, and every pixel has the same
-// winding number: the winding number changes only across an edge, none
-// crosses the wave's rectangle, and for such edges the fp32 crossing test at
-// each pixel gives the geometric side (see kCullFarCrossExact).  `first`
-// holds the masks of the first 64 edges and `w0` their far_winding (computed
-// by the caller when first has no distance or exact crossing term): the
-// entry is far when no edge has a distance or exact crossing term.  For a
-// fill, `winding` receives the winding number of the wave's pixels.  Only a
-// closed chain's crossing count is the same on every row of the wave: an
-// open chain filled (no closing edge; a ring whose segments' shared end
-// points an optimizer moved apart is one) changes it between rows where one
-// of its edges ends right of the wave, so such entries take the edge walk,
-// whose far edges count per row (row_cross_term).  (Comparing the counts of
-// all eight rows instead was measured: slower than the edge walk.)
+// Then no pixel needs the exact coverage, and a pixel's winding number is the
+// sum of the right edges' terms on its row (ChunkMasks).  Returns true when
+// that sum is also the same on all eight rows (always so for a closed chain,
+// whose winding number changes only across an edge; a chain that is open by a
+// gap has rows beside the gap that differ, and takes the general path, which
+// then visits no edge).  `winding` receives it.  `first` holds the masks of
+// the first 64 edges.
 template <int MODE>
 __device__ __forceinline__ bool entry_far(const PrimRec& pr, const WaveRect& W,
                                           const EdgeCull* __restrict__ culls,
-                                          const ChunkMasks& first, int w0, int& winding) {
+                                          const ChunkMasks& first, int& winding) {
     if (first.dist | first.cross) return false;
-    if (MODE == 0 && !pr.closed) return false;
-    int w = MODE == 0 ? w0 : 0;
+    int w = 0;
+    if (MODE == 0) {
+        w = (int)(int8_t)first.right_lo;
+        // (Byte 0 is exact modulo 256, and so is the test: |w| <= 64.)
+        if (first.right_lo != w * 0x01010101 || first.right_hi != first.right_lo) return false;
+    }
     for (int c = pr.e0 + kWave; c < pr.e1; c += kWave) {
-        const int4 q = load_culls(culls, c, pr.e1);
-        const ChunkMasks m = chunk_masks<MODE == 0>(q, c, pr.e1, W);
+        const ChunkMasks m = chunk_masks<MODE == 0>(load_culls(culls, c, pr.e1), c, pr.e1, W);
         if (m.dist | m.cross) return false;
-        if (MODE == 0) w += far_winding(q, c, pr.e1, W);
+        if (MODE == 0) {
+            const int wc = (int)(int8_t)m.right_lo;
+            if (m.right_lo != wc * 0x01010101 || m.right_hi != m.right_lo) return false;
+            w += wc;
+        }
     }
     winding = w;
     return true;
@@ -748,8 +764,6 @@ __global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(
             // Everything this entry needs from its first cull words is taken
             // before the next entry's load reuses their registers.
             const ChunkMasks cm0 = chunk_masks<MODE == 0>(q_next, pr.e0, pr.e1, W);
-            const int w0 = (MODE == 0 && pr.closed && (cm0.dist | cm0.cross) == 0)
-                               ? far_winding(q_next, pr.e0, pr.e1, W) : 0;
             if (todo) {
                 const int pid2 = __builtin_amdgcn_readlane(pid_l, (int)__builtin_ctzll(todo));
                 q_next = load_culls(culls, prims[pid2].e0, prims[pid2].e1);
@@ -767,7 +781,7 @@ __global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(
             // Coverage of each pixel; one compositing site below for every
             // path (so the pixels' state stays in the same registers).
             float cov[kPix];
-            if (entry_far<MODE>(pr, W, culls, cm0, w0, wnd)) {
+            if (entry_far<MODE>(pr, W, culls, cm0, wnd)) {
                 // Uniform entry: outside (nothing to do) or, for a fill whose
                 // winding number says inside, coverage 1 at every pixel.
                 bool inside_all = false;
@@ -844,7 +858,10 @@ __global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(
                 }
                 // The log record of this entry and wave: inside and exact bits, and
                 // each exact pixel's best edge and coverage, for the backward.
-                if (LOG) {
+                if (LOG && (in0 & in1) == ~0ull && nx == 0) {
+                    idx_l = lane == k ? kLogInside : idx_l;   // coverage 1, no record
+                    logged |= 1ull << k;
+                } else if (LOG) {
                     const uint32_t units = kLogHeaderUnits + (uint32_t)((nx + 1) >> 1);
                     if (st.n + units > kLogStageUnits) log_flush(log_pool, stage, st);
                     const int32_t at = log_reserve(log_ctr, log_first, log_units, lc, units);
