@@ -19,6 +19,8 @@
 // scalar instructions; its edges are tested lane-parallel (one edge per lane,
 // one ballot per test), and the wave then evaluates only the edges that can
 // matter.  Results stay bit-identical to evaluating every edge.
+#include <type_traits>
+
 #include "cs_common.h"
 #include "../../include/cubicsplat_hip.h"
 
@@ -438,9 +440,21 @@ __host__ __device__ __forceinline__ int order_cap(int n) {
 struct SubBlock {
     int index;  // sub-block (the unit of the tile order and the wave costs), -1: none
     int tile;   // its tile
-    int slot;   // this wave's slot among the tile's waves
+    int slot;   // the 16 x 8 block's slot among those of the tile
     int r0, c0; // its first pixel row and column
 };
+
+__device__ __forceinline__ SubBlock sub_block_at(const TileGrid& tg, int index, int half) {
+    SubBlock b;
+    b.index = index;
+    const int sy = b.index / tg.sbtx, sx = b.index - sy * tg.sbtx;
+    const int ty = sy / tg.sby, tx = sx / tg.sbx;
+    b.tile = ty * tg.tbx + tx;
+    b.slot = 2 * ((sy - ty * tg.sby) * tg.sbx + (sx - tx * tg.sbx)) + half;
+    b.r0 = sy * kTile;
+    b.c0 = sx * kTile;
+    return b;
+}
 
 // Sub-block of workgroup b: with a heavy-first order (cs_raster_tile_order,
 // 8 ocap positions; the launch has 8 ocap workgroups, workgroup b on XCD
@@ -450,18 +464,78 @@ struct SubBlock {
 // independent.
 __device__ __forceinline__ SubBlock sub_block(const TileGrid& tg,
                                               const int32_t* __restrict__ tile_order, int wv) {
-    SubBlock b;
-    b.index = tile_order
-                  ? __builtin_amdgcn_readfirstlane(
-                        tile_order[(blockIdx.x & 7) * tg.ocap + (blockIdx.x >> 3)])
-                  : xcd_tile(blockIdx.x, tg.nsb);
-    const int sy = b.index / tg.sbtx, sx = b.index - sy * tg.sbtx;
-    const int ty = sy / tg.sby, tx = sx / tg.sbx;
-    b.tile = ty * tg.tbx + tx;
-    b.slot = 2 * ((sy - ty * tg.sby) * tg.sbx + (sx - tx * tg.sbx)) + wv;
-    b.r0 = sy * kTile;
-    b.c0 = sx * kTile;
-    return b;
+    return sub_block_at(tg,
+                        tile_order
+                            ? __builtin_amdgcn_readfirstlane(
+                                  tile_order[(blockIdx.x & 7) * tg.ocap + (blockIdx.x >> 3)])
+                            : xcd_tile(blockIdx.x, tg.nsb),
+                        wv);
+}
+
+// Split launches (small images): NW waves on each 16 x 8 block of pixels, one
+// workgroup per block, the two blocks of a sub-block on the same XCD.
+//
+// A launch of one wave per block leaves most of the chip idle when the image
+// is small, and each wave then walks its list at the latency of one entry
+// after the other (a 128 x 128 image has 128 blocks for 1024 SIMDs).  Here the
+// waves of a block take one entry each, NW at a time: the entry's coverage
+// (forward) or gradients (backward) depend on the pixels' geometry alone, and
+// only the short recurrence over the transmittance is serial.  Each wave
+// leaves its entry's alpha and colour in LDS; after a barrier every wave runs
+// that recurrence over the NW entries for itself (about 12 vector operations
+// an entry and pixel, the same operations in the same order as one wave would
+// run, so the results are bit-identical), so no state is handed back.
+// Training step of 64 paths at 128 x 128: forward 135 -> 32 us, backward
+// 73 -> 22 us; the rule is at split_waves.
+__device__ __forceinline__ SubBlock split_block(const TileGrid& tg,
+                                                const int32_t* __restrict__ tile_order) {
+    if (tile_order) {
+        const int q = blockIdx.x >> 3;
+        return sub_block_at(tg,
+                            __builtin_amdgcn_readfirstlane(
+                                tile_order[(blockIdx.x & 7) * tg.ocap + (q >> 1)]),
+                            q & 1);
+    }
+    const int i = xcd_tile(blockIdx.x, 2 * tg.nsb);
+    return sub_block_at(tg, i >> 1, i & 1);
+}
+
+// Waves per block of a launch over nsb sub-blocks (1: not split).  A launch
+// that leaves the chip idle takes as long as its longest list; splitting
+// shortens that, but every wave repeats the cull tests and the recurrence,
+// which costs more than it saves once the launch fills the chip.  Measured
+// (us, one, 4 and 8 waves; fills at one path per 400 pixels, strokes at one
+// per 67), forward and backward:
+//   sub-blocks    fill forward     fill backward    stroke forward   stroke backward
+//        64     46 / 28 / 19     33 / 27 / 25     54 / 28 / 20     65 / 40 / 34
+//       475     64 / 44 / 40     47 / 33 / 37     74 / 39 / 35     84 / 47 / 50
+//      1024     71 / 64 / 71     58 / 51 / 64     78 / 53 / 55     89 / 62 / 76
+//      1536     76 / 79 / 96     59 / 61 / 83     84 / 65 / 74     96 / 76 / 98
+//      2565     80 / 103 / 140   67 / 81 / 114    93 / 91 / 113    105 / 102 / 145
+// (16 waves are no faster at 64 and slower from 256 on; two waves gain
+// little at 950 and nothing at 1536.)
+__host__ __forceinline__ int split_waves(int mode, int nsb) {
+    return nsb <= 512 ? 8 : nsb <= (mode == 0 ? 1152 : 2304) ? 4 : 1;
+}
+
+// One entry of a split round, left in LDS for the block's waves: its alpha at
+// each pixel, its colour and list index, and whether it contributes at all.
+// Two buffers in turn, so one barrier a round is enough: a wave writes buffer
+// b again two rounds later, after a barrier that every wave reaches only when
+// it has read b.
+template <int NW>
+struct SplitRound {
+    float alpha[2][NW][kPix * kWave];
+    float4 col[2][NW];
+    int used[2][NW];
+};
+
+// Barrier over the workgroup's LDS accesses alone (global loads issued ahead
+// stay in flight).
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // A wave's duration in ticks of the constant 100 MHz clock, stored in its
@@ -941,6 +1015,264 @@ __global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(
     record_wave_cost(kt->wave_cost, sb.index, t_start);
 }
 
+// What a wave of the split forward holds of its next entry: the first 64
+// edges' cull words and geometry, lane k edge e0 + k, loaded a round ahead.
+struct SplitEdges {
+    int4 q;
+    float4 a, b;
+};
+
+__device__ __forceinline__ SplitEdges split_load(const EdgeCull* __restrict__ culls,
+                                                 const EdgeRec* __restrict__ edges, int c,
+                                                 int e1) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int e = max(min(c + lane, e1 - 1), 0);
+    SplitEdges r;
+    r.q = *reinterpret_cast<const int4*>(culls + e);
+    const float4* p = reinterpret_cast<const float4*>(edges + e);
+    r.a = p[0];
+    r.b = p[1];
+    return r;
+}
+
+// chunk_geometry with the edges' geometry in the lanes' registers instead of
+// scalar memory: the wave puts it in LDS and reads each edge it visits from
+// there, one ahead.
+template <bool CROSS>
+__device__ __forceinline__ void split_chunk(const SplitEdges& r, int c, int e1, const WaveRect& W,
+                                            float4* __restrict__ stage, float px,
+                                            const float (&py)[kPix], Geom (&G)[kPix]) {
+    const ChunkMasks cm = chunk_masks<CROSS>(r.q, c, e1, W);
+    uint64_t todo = cm.dist | cm.cross;
+    if (todo) {
+        const int lane = threadIdx.x & (kWave - 1);
+        stage[2 * lane] = r.a;
+        stage[2 * lane + 1] = r.b;
+        int k = (int)__builtin_ctzll(todo);
+        float4 a = stage[2 * k], b = stage[2 * k + 1];
+        while (todo) {
+            todo &= todo - 1;
+            const EdgeRec E{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            const int kc = k;
+            k = todo ? (int)__builtin_ctzll(todo) : 0;
+            a = stage[2 * k];
+            b = stage[2 * k + 1];
+            const bool near = (cm.dist >> kc) & 1, cross = CROSS && ((cm.cross >> kc) & 1);
+            const float wx = px - E.x0;
+#pragma unroll
+            for (int p = 0; p < kPix; ++p) {
+                const float wy = py[p] - E.y0;
+                if (near) dist_term<1>(E, c + kc, wx, wy, G[p]);
+                if (cross) cross_term(E, wx, wy, py[p], G[p]);
+            }
+        }
+    }
+    if constexpr (CROSS) {
+        if (cm.right_lo | cm.right_hi) {
+            G[0].winding += row_term(cm.right_lo);
+            G[1].winding += row_term(cm.right_hi);
+        }
+    }
+}
+
+// The forward of a split launch (see split_block): the arguments, results and
+// log of k_raster_fwd.  The block's log region is shared by its waves through
+// an LDS cursor; a record that does not fit there goes to blocks that its wave
+// reserves, as in k_raster_fwd.
+template <int MODE, bool LOG, int NW>
+__global__ __launch_bounds__(kWave * NW) void k_raster_fwd_split(
+    FwdTail tail, const int32_t* __restrict__ prim_ids_g, const int32_t* __restrict__ bins,
+    const EdgeRec* __restrict__ edges_g, const EdgeCull* __restrict__ culls,
+    const PrimRec* __restrict__ prims_g, TileGrid tg, const int32_t* __restrict__ tile_order,
+    int32_t* __restrict__ log_index, uint4* __restrict__ log_pool, uint32_t* __restrict__ log_ctr,
+    uint32_t log_first, uint32_t log_units, uint32_t log_per_entry) {
+    const uint64_t t_start = __builtin_amdgcn_s_memrealtime();
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const SubBlock sb = split_block(tg, tile_order);
+    if (sb.index < 0) return;  // a position past this XCD's run (whole workgroup)
+    const int half = sb.slot & 1;
+    const int r0 = sb.r0 + half * kWaveRows;
+    const LanePixels L = lane_pixels(r0, sb.c0, tail.img_h, tail.img_w);
+    const WaveRect W{sb.c0, sb.c0 + kTile - 1, r0, r0 + kWaveRows - 1};
+    const cptr<PrimRec> prims = as_const(prims_g);
+    const int g0 = bins[2 * sb.tile], g1 = bins[2 * sb.tile + 1];
+    float T[kPix], C0[kPix], C1[kPix], C2[kPix];
+    int cur[kPix];
+    bool done[kPix];
+#pragma unroll
+    for (int p = 0; p < kPix; ++p) {
+        T[p] = 1.0f;
+        C0[p] = C1[p] = C2[p] = 0.0f;
+        cur[p] = 0;
+        done[p] = !L.in_img[p];
+    }
+    __shared__ SplitRound<NW> round;
+    __shared__ float4 stage_all[NW][2 * kWave];
+    __shared__ uint32_t cursor;
+    float4* const stage = stage_all[wv];
+    const uint32_t region = (uint32_t)(g1 - g0) * log_per_entry;
+    const uint32_t own = 1u + (uint32_t)tg.waves * (uint32_t)g0 * log_per_entry +
+                         (uint32_t)sb.slot * region;
+    LogCursor lc{0u, 0u, false};
+    if (LOG && threadIdx.x == 0) cursor = 0u;   // (read after the first barrier)
+    lds_barrier();
+    int buf = 0;
+    bool finished = false;
+    for (int gc = g0; gc < g1 && !finished; gc += kWave) {
+        const int gl = gc + lane;
+        const bool in_list = gl < g1;
+        const int pid_l = in_list ? prim_ids_g[gl] : 0;
+        const int2 er_l = *reinterpret_cast<const int2*>(&prims_g[pid_l].e0);
+        const bool keep = in_list && !prim_culled_lane<MODE>(prims_g + pid_l, W);
+        const uint64_t todo = __ballot(keep);
+        const int rank = lane_rank(todo), ns = __builtin_popcountll(todo);
+        int idx_l = kLogEmpty;
+        uint64_t logged = 0;
+        // This wave's entries of the chunk: those of rank wv, wv + NW, ...
+        uint64_t at_rank = __ballot(keep && rank == wv);
+        SplitEdges next{};
+        if (at_rank) {
+            const int k = (int)__builtin_ctzll(at_rank);
+            next = split_load(culls, edges_g, __builtin_amdgcn_readlane(er_l.x, k),
+                              __builtin_amdgcn_readlane(er_l.y, k));
+        }
+        for (int base = 0; base < ns; base += NW) {
+            bool any_live = false;
+#pragma unroll
+            for (int p = 0; p < kPix; ++p) any_live |= !done[p];
+            if (__ballot(any_live) == 0) {   // the same in every wave of the block
+                finished = true;
+                break;
+            }
+            buf ^= 1;
+            const int cnt = min(NW, ns - base);
+            if (wv < cnt) {
+                const int k = (int)__builtin_ctzll(at_rank);
+                const int pid = __builtin_amdgcn_readlane(pid_l, k);
+                const PrimRec pr = load_prim_fwd(prims, pid);
+                Geom G[kPix];
+#pragma unroll
+                for (int p = 0; p < kPix; ++p) {
+                    G[p].min_d2 = 1e30f;
+                    G[p].winding = 0;
+                    G[p].best = -1;
+                }
+                const SplitEdges here = next;
+                at_rank = __ballot(keep && rank == base + NW + wv);
+                if (at_rank) {
+                    const int k2 = (int)__builtin_ctzll(at_rank);
+                    next = split_load(culls, edges_g, __builtin_amdgcn_readlane(er_l.x, k2),
+                                      __builtin_amdgcn_readlane(er_l.y, k2));
+                }
+                split_chunk<MODE == 0>(here, pr.e0, pr.e1, W, stage, L.px, L.py, G);
+                for (int c = pr.e0 + kWave; c < pr.e1; c += kWave)
+                    split_chunk<MODE == 0>(split_load(culls, edges_g, c, pr.e1), c, pr.e1, W,
+                                           stage, L.px, L.py, G);
+                const float D2 = pr.cull_d * pr.cull_d, D2o = pr.cull_out * pr.cull_out;
+                bool ex[kPix], ins[kPix];
+                float cov[kPix];
+#pragma unroll
+                for (int p = 0; p < kPix; ++p) {
+                    ins[p] = inside_of<MODE>(pr, G[p]);
+                    ex[p] = !done[p] && !(G[p].min_d2 > (ins[p] ? D2 : D2o));
+                    cov[p] = ins[p] ? 1.0f : 0.0f;
+                    if (ex[p]) cov[p] = exact_coverage<MODE>(pr, G[p].min_d2, ins[p]);
+                    round.alpha[buf][wv][p * kWave + lane] =
+                        fminf(kAlphaCap, pr.opacity * cov[p]);
+                }
+                const uint64_t x0 = __ballot(ex[0]), x1 = __ballot(ex[1]);
+                const uint64_t in0 = MODE == 0 ? (uint64_t)__ballot(ins[0]) : 0ull;
+                const uint64_t in1 = MODE == 0 ? (uint64_t)__ballot(ins[1]) : 0ull;
+                const bool some = (in0 | in1 | x0 | x1) != 0;
+                if (lane == 0) {
+                    round.col[buf][wv] =
+                        make_float4(pr.r, pr.g, pr.b, __builtin_bit_cast(float, gc + k));
+                    round.used[buf][wv] = (int)some;
+                }
+                if (LOG) {
+                    int32_t at = some ? kLogInside : kLogEmpty;
+                    if (some && !((in0 & in1) == ~0ull && (x0 | x1) == 0)) {
+                        const int n0 = __builtin_popcountll(x0);
+                        const uint32_t units =
+                            kLogHeaderUnits +
+                            (uint32_t)((n0 + __builtin_popcountll(x1) + 1) >> 1);
+                        uint32_t c = 0;
+                        if (lane == 0) c = atomicAdd(&cursor, units);
+                        c = __builtin_amdgcn_readfirstlane(c);
+                        at = c + units <= region
+                                 ? (int32_t)(own + c)
+                                 : log_reserve(log_ctr, log_first, log_units, lc, units);
+                        if (at >= 0) {
+                            uint4* const rec = log_pool + at;
+                            if (lane == 0) {
+                                rec[0] = make_uint4((uint32_t)in0, (uint32_t)(in0 >> 32),
+                                                    (uint32_t)in1, (uint32_t)(in1 >> 32));
+                                rec[1] = make_uint4((uint32_t)x0, (uint32_t)(x0 >> 32),
+                                                    (uint32_t)x1, (uint32_t)(x1 >> 32));
+                            }
+                            int2* pairs = reinterpret_cast<int2*>(rec + kLogHeaderUnits);
+                            if (ex[0])
+                                pairs[lane_rank(x0)] =
+                                    make_int2(G[0].best, __builtin_bit_cast(int, cov[0]));
+                            if (ex[1])
+                                pairs[n0 + lane_rank(x1)] =
+                                    make_int2(G[1].best, __builtin_bit_cast(int, cov[1]));
+                        }
+                    }
+                    idx_l = lane == k ? at : idx_l;
+                    logged |= 1ull << k;
+                }
+            }
+            lds_barrier();
+            const int u = lane < cnt ? round.used[buf][lane] : 0;
+            for (uint64_t m = __ballot(u != 0); m; m &= m - 1) {
+                const int j = (int)__builtin_ctzll(m);
+                const float4 col = round.col[buf][j];
+                PrimRec pr{};
+                pr.r = col.x;
+                pr.g = col.y;
+                pr.b = col.z;
+#pragma unroll
+                for (int p = 0; p < kPix; ++p)
+                    composite(pr, round.alpha[buf][j][p * kWave + lane],
+                              __builtin_bit_cast(int, col.w), T[p], C0[p], C1[p], C2[p], cur[p],
+                              done[p]);
+            }
+        }
+        if ((logged >> lane) & 1u) log_index[(size_t)tg.waves * gl + sb.slot] = idx_l;
+    }
+    // Every wave holds the block's pixels; wave 0 writes them.
+    if (wv == 0) {
+        const size_t np = (size_t)tail.img_h * tail.img_w;
+        const size_t ch = tail.out_planar ? np : 1;
+        const float bg0 = tail.bg[0], bg1 = tail.bg[1], bg2 = tail.bg[2];
+#pragma unroll
+        for (int p = 0; p < kPix; ++p) {
+            if (!L.in_img[p]) continue;
+            const size_t pix = (size_t)L.i[p] * tail.img_w + L.j;
+            tail.final_T[pix] = T[p];
+            tail.final_idx[pix] = cur[p];
+            const float o0 = __builtin_fmaf(T[p], bg0, C0[p]);
+            const float o1 = __builtin_fmaf(T[p], bg1, C1[p]);
+            const float o2 = __builtin_fmaf(T[p], bg2, C2[p]);
+            float* const o = tail.out + (tail.out_planar ? pix : 3 * pix);
+            o[0] = o0;
+            o[ch] = o1;
+            o[2 * ch] = o2;
+            if (tail.out_planes) {
+                tail.out_planes[pix] = o0;
+                tail.out_planes[np + pix] = o1;
+                tail.out_planes[2 * np + pix] = o2;
+            }
+        }
+        if (tail.wave_cost && lane == 0) {
+            const uint64_t dt = __builtin_amdgcn_s_memrealtime() - t_start;
+            tail.wave_cost[2 * sb.index + half] = dt > 0xffffffffull ? 0xffffffffu : (uint32_t)dt;
+        }
+    }
+}
+
 // First unit of the log pool: the counter of the shared blocks, which start
 // after the waves' own regions.
 __global__ void k_log_init(uint4* __restrict__ pool, uint32_t first_shared) {
@@ -1019,6 +1351,7 @@ struct GradRec {
     float v;
 };
 constexpr uint32_t kGradBufRecs = 256;   // 4 KiB of LDS per wave
+constexpr uint32_t kGradBufRecsSplit = 128;
 
 // Per-primitive gradients (colour, opacity, inverse variance, stroke width)
 // go, when the caller gives a scratch buffer, to one of kGradReplicas copies
@@ -1088,7 +1421,8 @@ __global__ __launch_bounds__(256) void k_prim_rep_finalize(
 
 struct GradBuf {
     GradRec* rec;
-    uint32_t n;   // wave-uniform
+    uint32_t n;     // wave-uniform
+    uint32_t cap;   // (a constant of the kernel)
 };
 
 __device__ __forceinline__ void grad_flush(GradBuf& gb) {
@@ -1105,7 +1439,7 @@ __device__ __forceinline__ void grad_flush(GradBuf& gb) {
 // Records (dst, v) from the lanes with `add` (lanes 8..15 after
 // wave_reduce8, each its slot); eight records per call.
 __device__ __forceinline__ void grad_push8(GradBuf& gb, bool add, float* dst, float v) {
-    if (gb.n + 8 > kGradBufRecs) grad_flush(gb);
+    if (gb.n + 8 > gb.cap) grad_flush(gb);
     const int lane = threadIdx.x & (kWave - 1);
     if (lane >= 8 && lane < 16) gb.rec[gb.n + (lane - 8)] = GradRec{add ? dst : nullptr, v};
     gb.n += 8;
@@ -1131,8 +1465,13 @@ __device__ __forceinline__ void grad_push8(GradBuf& gb, bool add, float* dst, fl
 // fit its scalar registers; the general instance keeps about 40 of them in
 // vector-register lanes, and each reload is a vector instruction (config 3
 // backward 92.5 -> 82.7 us).
-template <int MODE, bool COUNT, bool ADAPTIVE, bool LEAN>
-__global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(7))) void k_raster_bwd(
+// NW > 1: a split launch (split_block), NW waves per 16 x 8 block.  Each wave
+// then takes one of the NW entries of a round; the pixels' state is advanced
+// over the whole round in every wave, and a wave's own entry is given the
+// state that the one-wave walk would have reached there.
+template <int MODE, bool COUNT, bool ADAPTIVE, bool LEAN, int NW>
+__global__ __launch_bounds__(NW > 1 ? kWave * NW : kRasterThreads)
+__attribute__((amdgpu_waves_per_eu(NW > 1 ? 4 : 7))) void k_raster_bwd(
     const int32_t* __restrict__ prim_ids_g, const int32_t* __restrict__ bins,
     const EdgeRec* __restrict__ edges_g, const EdgeCull* __restrict__ culls,
     const PrimRec* __restrict__ prims_g, const float* __restrict__ bg, int img_h, int img_w,
@@ -1146,13 +1485,14 @@ __global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(
     unsigned long long* __restrict__ counts) {
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const SubBlock sb = sub_block(tg, tile_order, wv);
+    SubBlock sb;
+    if constexpr (NW > 1) sb = split_block(tg, tile_order);
+    else sb = sub_block(tg, tile_order, wv);
     if (sb.index < 0) return;  // a position past this XCD's run (whole workgroup)
     const int tile = sb.tile;
-    const int r0 = sb.r0 + wv * kWaveRows;
+    const int r0 = sb.r0 + (NW > 1 ? (sb.slot & 1) : wv) * kWaveRows;
     const LanePixels L = lane_pixels(r0, sb.c0, img_h, img_w);
     const WaveRect W{sb.c0, sb.c0 + kTile - 1, r0, r0 + kWaveRows - 1};
-    const cptr<int32_t> prim_ids = as_const(prim_ids_g);
     const cptr<PrimRec> prims = as_const(prims_g);
     const int g0 = bins[2 * tile], g1 = bins[2 * tile + 1];
     const float bg0 = bg[0], bg1 = bg[1], bg2 = bg[2];
@@ -1186,21 +1526,34 @@ __global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(
     const int gstart = min(g1 - 1, __builtin_amdgcn_readfirstlane(wave_max_i(fmax)));
     const int slot = reduce8_slot(lane & 7);
     const bool adder = (lane & ~7) == 8;
-    __shared__ GradRec grad_rec_all[kRasterThreads / kWave][kGradBufRecs];
+    constexpr int kWaves = NW > 1 ? NW : kRasterThreads / kWave;
+    constexpr uint32_t kRecs = NW > 1 ? kGradBufRecsSplit : kGradBufRecs;
+    __shared__ GradRec grad_rec_all[kWaves][kRecs];
     // Uniform flattening with at most kBasisTable edges per segment: the
     // accumulation weights at t = e / eps for every e, computed once per
     // workgroup with seg_basis (so the same values) and read per pixel.
     __shared__ float4 basis_tab[kBasisTable + 1];
     const bool use_tab = !ADAPTIVE && eps <= kBasisTable;
     if (use_tab) {
-        for (int e = (int)threadIdx.x; e <= eps; e += kRasterThreads) {
+        for (int e = (int)threadIdx.x; e <= eps; e += kWaves * kWave) {
             float bb[4];
             seg_basis(e, inv_e, bb);
             basis_tab[e] = make_float4(bb[0], bb[1], bb[2], bb[3]);
         }
         __syncthreads();
     }
-    GradBuf gbuf{grad_rec_all[wv], 0u};
+    GradBuf gbuf{grad_rec_all[wv], 0u, kRecs};
+    // (Split launches) the round's entries, and the state after the round.
+    __shared__ typename std::conditional<(NW > 1), SplitRound<NW>, int>::type round;
+    float Tn[kPix], n0[kPix], n1[kPix], n2[kPix];
+    int buf = 0;
+    if constexpr (NW > 1) {
+#pragma unroll
+        for (int p = 0; p < kPix; ++p) {
+            Tn[p] = T[p];
+            n0[p] = n1[p] = n2[p] = 0.0f;
+        }
+    }
     // Entries from gstart down to g0 in chunks of 64: lane k tests entry
     // gc - k with the forward's primitive cull, and the wave visits the
     // survivors in descending order -- exactly the entries the forward
@@ -1225,18 +1578,31 @@ __global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(
           hb = log_pool[at_l + 1];
       }
       uint64_t todo = __ballot(kept && at_l != kLogEmpty);
-      while (todo) {
-        const int k = (int)__builtin_ctzll(todo);
-        todo &= todo - 1;
+      // (Split) the lane's rank among the chunk's entries, and the round's first.
+      const int rank = NW > 1 ? lane_rank(todo) : 0;
+      const int ns = NW > 1 ? __builtin_popcountll(todo) : 0;
+      for (int base = 0; NW > 1 ? base < ns : todo != 0; base += NW) {
+        int k;
+        bool have = true;   // (split) this wave has an entry in the round
+        if constexpr (NW > 1) {
+            have = base + wv < ns;
+            k = (int)__builtin_ctzll(__ballot(rank == base + wv && ((todo >> lane) & 1)) |
+                                     (1ull << 63));
+            buf ^= 1;
+        } else {
+            k = (int)__builtin_ctzll(todo);
+            todo &= todo - 1;
+        }
         const int g = gc - k;
         bool valid[kPix];
         bool any_valid = false;
 #pragma unroll
         for (int p = 0; p < kPix; ++p) {
-            valid[p] = L.in_img[p] & (g <= fidx[p]);
+            valid[p] = have & L.in_img[p] & (g <= fidx[p]);
             any_valid |= valid[p];
         }
-        if (__ballot(any_valid) == 0) continue;
+        if constexpr (NW > 1) have = have && __ballot(any_valid) != 0;
+        else if (__ballot(any_valid) == 0) continue;
         const int pid_cur = __builtin_amdgcn_readlane(pid_l, k);
         const PrimRec pr = prims[pid_cur];
         // The forward's log record of this entry and wave, if it has one
@@ -1255,7 +1621,16 @@ __global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(
         Geom G[kPix];
         bool exact[kPix];
         float lcov[kPix];
-        if (uniform_inside) {
+        if (NW > 1 && !have) {
+#pragma unroll
+            for (int p = 0; p < kPix; ++p) {
+                exact[p] = false;
+                lcov[p] = 0.0f;
+                G[p].winding = 0;
+                G[p].best = 0;
+                G[p].min_d2 = G[p].bproj = G[p].bdx = G[p].bdy = 0.0f;
+            }
+        } else if (uniform_inside) {
 #pragma unroll
             for (int p = 0; p < kPix; ++p) {
                 G[p].winding = 1;
@@ -1319,6 +1694,55 @@ __global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
             for (int p = 0; p < kPix; ++p) ex[p] = valid[p] && exact[p];
             n.cover += (uint64_t)wave_count(ex);
+        }
+        if constexpr (NW > 1) {
+            // The round: this wave's alpha (as below; 0 where the entry does
+            // not count), then the state at its entry and after the round.
+            if (have) {
+#pragma unroll
+                for (int p = 0; p < kPix; ++p) {
+                    const float cov = exact[p] ? lcov[p] : inside_of<MODE>(pr, G[p]) ? 1.0f : 0.0f;
+                    const float al = fminf(kAlphaCap, pr.opacity * cov);
+                    round.alpha[buf][wv][p * kWave + lane] =
+                        valid[p] && al >= kAlphaMin ? al : 0.0f;
+                }
+                if (lane == 0) round.col[buf][wv] = make_float4(pr.r, pr.g, pr.b, 0.0f);
+            }
+            if (lane == 0) round.used[buf][wv] = (int)have;
+            lds_barrier();
+#pragma unroll
+            for (int p = 0; p < kPix; ++p) {
+                T[p] = Tn[p];
+                b0[p] = n0[p];
+                b1[p] = n1[p];
+                b2[p] = n2[p];
+            }
+            const int u = lane < NW ? round.used[buf][lane] : 0;
+            for (uint64_t m = __ballot(u != 0); m; m &= m - 1) {
+                const int j = (int)__builtin_ctzll(m);
+                if (j == wv) {
+#pragma unroll
+                    for (int p = 0; p < kPix; ++p) {
+                        T[p] = Tn[p];
+                        b0[p] = n0[p];
+                        b1[p] = n1[p];
+                        b2[p] = n2[p];
+                    }
+                }
+                const float4 col = round.col[buf][j];
+#pragma unroll
+                for (int p = 0; p < kPix; ++p) {
+                    const float al = round.alpha[buf][j][p * kWave + lane];
+                    const bool take = al > 0.0f;
+                    const float Tj = Tn[p] * grad_rcp(1.0f - al);
+                    const float fac = al * Tj;
+                    Tn[p] = take ? Tj : Tn[p];
+                    n0[p] = take ? __builtin_fmaf(col.x, fac, n0[p]) : n0[p];
+                    n1[p] = take ? __builtin_fmaf(col.y, fac, n1[p]) : n1[p];
+                    n2[p] = take ? __builtin_fmaf(col.z, fac, n2[p]) : n2[p];
+                }
+            }
+            if (!have) continue;
         }
         // Per-primitive sums over the lane's pixels: v_r, v_g, v_b, v_opacity,
         // v_inv_sigma2, v_stroke; contribution sums r, g, b, r + g + b.
@@ -2093,10 +2517,28 @@ static unsigned raster_groups(const RasterArgs& a) {
     return (unsigned)(a.order ? 8 * a.tg.ocap : a.tg.nsb);
 }
 
+// Workgroups of a split launch: one per 16 x 8 block (or position of an order).
+static unsigned split_groups(const RasterArgs& a) { return 2 * raster_groups(a); }
+
+template <int MODE, int NW>
+static void launch_fwd_split(const RasterArgs& a, const FwdTail& tail) {
+    auto kern = a.log_index ? k_raster_fwd_split<MODE, true, NW> : k_raster_fwd_split<MODE, false, NW>;
+    hipLaunchKernelGGL(kern, dim3(split_groups(a)), dim3(kWave * NW), 0, a.stream, tail, a.ids,
+                       a.bins, a.E, a.C, a.P, a.tg, a.order, a.log_index, a.log_pool, a.log_ctr,
+                       a.log_first, a.log_units, a.log_per_entry);
+}
+
 template <int MODE, bool COUNT>
 static void launch_fwd(const RasterArgs& a) {
     const FwdTail tail{a.bg,        a.out,    a.out_planes, a.final_T, a.final_idx,
                        a.wave_cost, a.counts, a.out_planar, a.img_h,   a.img_w};
+    if constexpr (!COUNT) {
+        switch (split_waves(MODE, a.tg.nsb)) {
+            case 8: return launch_fwd_split<MODE, 8>(a, tail);
+            case 4: return launch_fwd_split<MODE, 4>(a, tail);
+            default: break;
+        }
+    }
     auto kern = a.log_index ? k_raster_fwd<MODE, COUNT, true> : k_raster_fwd<MODE, COUNT, false>;
     hipLaunchKernelGGL(kern, dim3(raster_groups(a)), dim3(kRasterThreads), 0,
                        a.stream, tail, a.ids, a.bins, a.E, a.C, a.P, a.img_h, a.img_w, a.tg,
@@ -2104,19 +2546,29 @@ static void launch_fwd(const RasterArgs& a) {
                        a.log_per_entry);
 }
 
-template <int MODE, bool COUNT, bool ADAPTIVE, bool LEAN>
-static void launch_bwd4(const RasterArgs& a) {
+template <int MODE, bool COUNT, bool ADAPTIVE, bool LEAN, int NW>
+static void launch_bwd5(const RasterArgs& a) {
     // ceil(2^32 / eps) for div_eps (unused when eps <= 1).
     const uint32_t magic =
         a.eps > 1 ? (uint32_t)((0x100000000ull + (uint64_t)(a.eps - 1)) / (uint64_t)a.eps) : 0u;
-    hipLaunchKernelGGL((k_raster_bwd<MODE, COUNT, ADAPTIVE, LEAN>), dim3(raster_groups(a)),
-                       dim3(kRasterThreads), 0, a.stream, a.ids, a.bins, a.E, a.C, a.P, a.bg,
+    hipLaunchKernelGGL((k_raster_bwd<MODE, COUNT, ADAPTIVE, LEAN, NW>),
+                       dim3(NW > 1 ? split_groups(a) : raster_groups(a)),
+                       dim3(NW > 1 ? kWave * NW : kRasterThreads), 0, a.stream, a.ids, a.bins, a.E, a.C, a.P, a.bg,
                        a.img_h, a.img_w, a.tg, a.order, a.eps, magic, a.aux, a.log_index,
                        a.log_pool, a.fT, a.fidx,
                        a.v_out, a.v_planar,
                        a.v_cub, a.v_col,
                        a.v_op, a.v_is2, a.v_sw, a.c_rgb, a.c_isect, a.prim_rep, a.nprim,
                        a.counts);
+}
+
+template <int MODE, bool COUNT, bool ADAPTIVE, bool LEAN>
+static void launch_bwd4(const RasterArgs& a) {
+    switch (COUNT ? 1 : split_waves(MODE, a.tg.nsb)) {
+        case 8: launch_bwd5<MODE, COUNT, ADAPTIVE, LEAN, COUNT ? 1 : 8>(a); break;
+        case 4: launch_bwd5<MODE, COUNT, ADAPTIVE, LEAN, COUNT ? 1 : 4>(a); break;
+        default: launch_bwd5<MODE, COUNT, ADAPTIVE, LEAN, 1>(a); break;
+    }
     if (a.prim_rep && a.fin_norm) {
         constexpr int NV = MODE == 1 ? 6 : 5;
         const int64_t n = (int64_t)a.nseg * 8 > (int64_t)a.nprim * NV ? (int64_t)a.nseg * 8
@@ -2435,6 +2887,10 @@ extern "C" int cs_rasterize_backward_counted(
                               v_stroke_widths, curve_contrib_rgb, curve_isect_contrib, nullptr,
                               log_index, log_pool, eval_counts, nprim, prim_scratch, tile_order,
                               stream);
+}
+
+extern "C" int32_t cs_raster_split_waves(int32_t nsub) {
+    return nsub > 0 ? split_waves(1, nsub) : 0;
 }
 
 extern "C" size_t cs_raster_tile_order_elems(int32_t ntiles) {

@@ -541,11 +541,13 @@ def log_layout(key, capacity: int, nsub: int, waves_per_tile: int = 2):
     """(units per entry, pool bytes) for a forward of scene shape `key` with
     `capacity` list entries and tiles of `waves_per_tile` waves: the waves'
     own regions, plus shared blocks for a quarter of them and one block per
-    wave (two per 16 x 16 sub-block)."""
+    launched wave (each 16 x 16 sub-block has two 16 x 8 blocks of
+    cs_raster_split_waves waves)."""
     _poll_log_use(key)
     units = _LOG_UNITS.get(key, LOG_FIRST_UNITS_PER_ENTRY)
     regions = 16 * waves_per_tile * capacity * units
-    shared = regions // 4 + 2 * nsub * N.RASTER_LOG_BLOCK_BYTES + (1 << 20)
+    waves = 2 * nsub * int(N.lib().cs_raster_split_waves(nsub))
+    shared = regions // 4 + waves * N.RASTER_LOG_BLOCK_BYTES + (1 << 20)
     return units, (16 + regions + shared + 255) // 256 * 256
 
 
