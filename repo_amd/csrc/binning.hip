@@ -724,7 +724,9 @@ __global__ __launch_bounds__(256) void k_split_half(const float* __restrict__ cu
 // Depth ranks of at most kRankPairsMax keys: one launch of all-pairs
 // counting.  Up to kRankSortMax: the first stage ranks each block of
 // kRankBlock keys among themselves (k_prim_prep does it for the cubic path,
-// k_rank_blocks for the others), the second merges the blocks.
+// k_gs_keys_rects for the Gaussians, k_rank_blocks for the others), the second
+// merges the blocks (k_rank_merge).  Up to kRankSegmentsMax: the blocks are
+// merged into segments, and those into the order.  Above, the radix sort.
 constexpr int kRankPairsMax = 8192;
 constexpr int kRankSortMax = 16384;
 constexpr int kRankBlock = 256;
@@ -1217,6 +1219,113 @@ __global__ __launch_bounds__(kMergeThreads) void k_rank_merge(
         order[pos] = i;
         rank_rects[pos] = rects[i];
     }
+}
+
+// More keys than one LDS holds (to kRankSegmentsMax): the sorted blocks are
+// merged in segments of kSegmentKeys in LDS, and a key's position is its
+// position in its segment plus, by binary search, the keys before it in every
+// other segment.  The searches read the segments from cache; a wave's 64 keys
+// are neighbours in their own segment's order, so after the first steps they
+// probe the same few lines.  Both launches are bound by the latency of their
+// search steps.  The four-pass radix sort that larger counts take runs 256
+// keys at a time per workgroup and is bound by its three barriers a step:
+// 24576 keys 98 -> 19 us, 100000 keys 109 -> 26 us (with the rectangles'
+// gather; and 4 us more in the launch that ranks the blocks).
+constexpr int kSegmentKeys = 4096;
+constexpr int kSegMergeWaves = 4;
+constexpr int kSegThreads = kWave * kSegMergeWaves;
+constexpr int kRankSegmentsMax = 1 << 18;
+constexpr int kSegmentBlocks = kSegmentKeys / kRankBlock;
+static_assert(kSegmentBlocks == 4 * kSegMergeWaves, "four blocks per wave, searched together");
+
+// 64 keys per workgroup, each wave a quarter of the segment's blocks (with
+// more keys per workgroup too few of the chip's LDS units work: 1024 keys took
+// 21 us at 24576 where 64 take 6.5).
+__global__ __launch_bounds__(kSegThreads) void k_rank_segments(
+    const uint32_t* __restrict__ keys, const uint32_t* __restrict__ sorted_keys,
+    const int32_t* __restrict__ block_rank, int n, uint32_t* __restrict__ seg_keys,
+    int32_t* __restrict__ seg_ids) {
+    __shared__ uint32_t sk[kSegmentKeys];
+    __shared__ int part[kSegMergeWaves][kWave];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int i = blockIdx.x * kWave + lane;
+    const int seg0 = blockIdx.x * kWave / kSegmentKeys * kSegmentKeys;
+    const int len = min(kSegmentKeys, n - seg0);
+    uint32_t v[kSegmentKeys / kSegThreads];
+#pragma unroll
+    for (int k = 0; k < kSegmentKeys / kSegThreads; ++k) {
+        const int j = k * kSegThreads + (int)threadIdx.x;
+        v[k] = j < len ? sorted_keys[seg0 + j] : 0u;
+    }
+    const bool ok = i < n;
+    const uint32_t ki = ok ? keys[i] : 0u;
+    const int br = ok ? block_rank[i] : 0;
+#pragma unroll
+    for (int k = 0; k < kSegmentKeys / kSegThreads; ++k)
+        sk[k * kSegThreads + threadIdx.x] = v[k];
+    __syncthreads();
+    const int own = (i - seg0) / kRankBlock, nblocks = (len + kRankBlock - 1) / kRankBlock;
+    int cnt = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int b = u * kSegMergeWaves + w, bb = min(b, nblocks - 1);
+        const int c = count_before(sk, bb * kRankBlock, min(kRankBlock, len - bb * kRankBlock), ki,
+                                   bb < own);
+        cnt += b < nblocks && b != own ? c : 0;
+    }
+    part[w][lane] = cnt;
+    __syncthreads();
+    if (w != 0 || !ok) return;
+    int pos = seg0 + br;
+#pragma unroll
+    for (int q = 0; q < kSegMergeWaves; ++q) pos += part[q][lane];
+    seg_keys[pos] = ki;
+    seg_ids[pos] = i;
+}
+
+__global__ __launch_bounds__(kSegThreads) void k_rank_segment_merge(
+    const uint32_t* __restrict__ seg_keys, const int32_t* __restrict__ seg_ids, int n,
+    const int4* __restrict__ rects, int32_t* __restrict__ order,
+    int4* __restrict__ rank_rects) {
+    __shared__ int part[kSegMergeWaves][kWave];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int j = blockIdx.x * kWave + lane;
+    const bool ok = j < n;
+    const uint32_t ki = seg_keys[min(j, n - 1)];
+    const int i = ok && w == 0 ? seg_ids[j] : 0;
+    const int4 rect = ok && w == 0 ? rects[i] : make_int4(0, 0, 0, 0);
+    const int own = blockIdx.x * kWave / kSegmentKeys;
+    const int nsegs = (n + kSegmentKeys - 1) / kSegmentKeys;
+    int cnt = 0;
+    // Wave w takes segments w, w + 4, ...; four searches per step.
+    for (int s0 = w; s0 < nsegs; s0 += 4 * kSegMergeWaves) {
+        int c[4] = {0, 0, 0, 0};
+        for (int step = kSegmentKeys; step >= 1; step >>= 1) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int s = min(s0 + u * kSegMergeWaves, nsegs - 1);
+                const int len = min(kSegmentKeys, n - s * kSegmentKeys);
+                const int probe = c[u] + step;
+                const uint32_t v = seg_keys[s * kSegmentKeys + min(probe, len) - 1];
+                if (probe <= len && (s < own ? v <= ki : v < ki)) c[u] = probe;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int s = s0 + u * kSegMergeWaves;
+            cnt += s < nsegs && s != own ? c[u] : 0;
+        }
+    }
+    part[w][lane] = cnt;
+    __syncthreads();
+    if (w != 0 || !ok) return;
+    int pos = j - own * kSegmentKeys;
+#pragma unroll
+    for (int q = 0; q < kSegMergeWaves; ++q) pos += part[q][lane];
+    order[pos] = i;
+    rank_rects[pos] = rect;
 }
 
 // Stable rank by counting, one wave per key, for at most kRankPairsMax keys:
@@ -1969,7 +2078,8 @@ extern "C" size_t cs_radix_counts_elems(int32_t n) {
     const int nb = blocks_for(n > 0 ? n : 1, kRsTile);
     const size_t radix = (size_t)256 * nb;
     // The sort of at most kRankSortMax keys stages 2n words here.
-    const size_t rank = n > kRankPairsMax && n <= kRankSortMax ? (size_t)2 * n : 0;
+    // (and so do the depth ranks of at most kRankSegmentsMax keys).
+    const size_t rank = n > kRankPairsMax && n <= kRankSegmentsMax ? (size_t)2 * n : 0;
     return radix > rank ? radix : rank;
 }
 
@@ -2057,6 +2167,17 @@ static int rank_and_count(bool blocks_ranked, uint32_t* keys, int32_t* order,
                            dim3(kMergeThreads), 0, stream, keys,
                            keys_alt, vals_alt, nprim, (const int32_t*)nullptr,
                            (uint32_t*)nullptr, (int32_t*)nullptr, prim_rects, order, rank_rects);
+    } else if (nprim <= kRankSegmentsMax) {
+        // Segment keys and ids in radix_counts [2 nprim].
+        int32_t* seg_ids = reinterpret_cast<int32_t*>(radix_counts + nprim);
+        if (!blocks_ranked)
+            hipLaunchKernelGGL(k_rank_blocks, dim3(blocks_for(nprim, kRankBlock)),
+                               dim3(kRankBlock), 0, stream, keys, nprim, keys_alt, vals_alt);
+        hipLaunchKernelGGL(k_rank_segments, dim3(blocks_for(nprim, kWave)), dim3(kSegThreads), 0,
+                           stream, keys, keys_alt, vals_alt, nprim, radix_counts, seg_ids);
+        hipLaunchKernelGGL(k_rank_segment_merge, dim3(blocks_for(nprim, kWave)),
+                           dim3(kSegThreads), 0, stream, radix_counts, seg_ids, nprim, prim_rects,
+                           order, rank_rects);
     } else {
         const int rc = cs_radix_sort_pairs_u32(keys, order, keys_alt, vals_alt, nprim, 32,
                                                radix_counts, scan_temp, stream);
@@ -2178,8 +2299,8 @@ static int bin_prepare(const float* cubics_norm, const int32_t* seg_offsets, con
                        adaptive ? seg_edge_offsets : nullptr, tbx, tby, mode, status,
                        prim_tile_ranges, num_tiles_hit, inv_sigma2s, keys, order,
                        reinterpret_cast<PrimRec*>(prim_recs),
-                       nprim <= kRankSortMax ? keys_alt : nullptr,
-                       nprim <= kRankSortMax ? vals_alt : nullptr);
+                       nprim <= kRankSegmentsMax ? keys_alt : nullptr,
+                       nprim <= kRankSegmentsMax ? vals_alt : nullptr);
     return rank_and_count(true, keys, order, reinterpret_cast<const int4*>(prim_tile_ranges),
                           reinterpret_cast<int4*>(rank_tile_ranges), nprim, tbx, tby, keys_alt,
                           vals_alt, radix_counts, scan_temp, tile_count,
@@ -2301,13 +2422,26 @@ __global__ __launch_bounds__(256) void k_gs_keys_rects(
     const float* __restrict__ xys, const float* __restrict__ conics,
     const int32_t* __restrict__ radii, const float* __restrict__ depths, int n, int bx, int by,
     int tbx, int tby, int4* __restrict__ rects, uint32_t* __restrict__ keys,
-    int32_t* __restrict__ order, int32_t* __restrict__ status) {
+    int32_t* __restrict__ order, int32_t* __restrict__ status,
+    uint32_t* __restrict__ block_sorted, int32_t* __restrict__ block_rank) {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g == 0) {
         status[0] = 0;
         status[1] = 0;
         status[2] = 0;
         status[3] = 0;
+    }
+    const uint32_t key = g < n ? __builtin_bit_cast(uint32_t, depths[g]) : 0xffffffffu;
+    if (block_sorted) {
+        // The first stage of the depth rank (as k_rank_blocks).
+        __shared__ uint4 ks[kRankBlock / 4];
+        reinterpret_cast<uint32_t*>(ks)[threadIdx.x] = key;
+        __syncthreads();
+        if (g < n) {
+            const int r = rank_in_block(ks, key, (int)threadIdx.x);
+            block_sorted[blockIdx.x * kRankBlock + r] = key;
+            block_rank[g] = r;
+        }
     }
     if (g >= n) return;
     int4 r = make_int4(0, 0, 0, 0);
@@ -2317,7 +2451,7 @@ __global__ __launch_bounds__(256) void k_gs_keys_rects(
         if ((r.z - r.x) * (r.w - r.y) <= 0) r = make_int4(0, 0, 0, 0);
     }
     rects[g] = r;
-    keys[g] = __builtin_bit_cast(uint32_t, depths[g]);
+    keys[g] = key;
     order[g] = g;
 }
 
@@ -2333,10 +2467,12 @@ extern "C" int cs_gs_bin_prepare(const float* xys, const float* conics, const in
         (reinterpret_cast<uintptr_t>(rank_tile_ranges) & 15) != 0)
         return CS_ERR_ARGS;
     const int tbx = (img_w + block_x - 1) / block_x, tby = (img_h + block_y - 1) / block_y;
+    const bool blocks = n > kRankPairsMax && n <= kRankSegmentsMax;
     hipLaunchKernelGGL(k_gs_keys_rects, dim3(blocks_for(n, 256)), dim3(256), 0, stream, xys,
                        conics, radii, depths, n, block_x, block_y, tbx, tby,
-                       reinterpret_cast<int4*>(tile_rects), keys, order, status);
-    return rank_and_count(false, keys, order, reinterpret_cast<const int4*>(tile_rects),
+                       reinterpret_cast<int4*>(tile_rects), keys, order, status,
+                       blocks ? keys_alt : nullptr, blocks ? vals_alt : nullptr);
+    return rank_and_count(blocks, keys, order, reinterpret_cast<const int4*>(tile_rects),
                           reinterpret_cast<int4*>(rank_tile_ranges), n, tbx, tby, keys_alt,
                           vals_alt, radix_counts, scan_temp, tile_count,
                           tile_scratch, status, stream);
