@@ -605,6 +605,185 @@ __global__ __launch_bounds__(kWave * kFlattenWaves) void k_project_flatten_wave(
     }
 }
 
+// Adaptive flattening for at most kDecasLaneDepth halvings, both passes with a
+// group of L = max(2, 2^maxd) lanes per segment instead of a thread (a thread
+// walks up to 2^maxd leaves from the root one after the other).  Bound by the
+// latency of the descent (a root and a division a level) and of the owner
+// search.  8192 segments, S = 24: counting 61 -> 8.8 us, writing 62 -> 11.3 us,
+// and a scan and a status launch (11 us) less.
+// Lane i descends from the root along the bits of i until its node is flat or
+// maxd deep, with the operations of decas_leaves, and so ends in the leaf that
+// holds the finest interval i; the leaf is the first such lane's.  The segments
+// are projected and staged as in k_project_flatten_wave.
+constexpr int kDecasLaneDepth = 6;
+// Segments per workgroup (as flatten_segs; the descent is the longer part).
+__host__ __device__ constexpr int decas_segs(int lanes) { return lanes >= 32 ? 16 : 32; }
+
+__device__ __forceinline__ int decas_slot(Cub& c, int maxd, float tol, uint32_t i) {
+    int d = 0;
+    while (d < maxd && !cub_flat(c, tol)) {
+        Cub l, r;
+        cub_split(c, l, r);
+        c = ((i >> (maxd - 1 - d)) & 1u) ? r : l;
+        ++d;
+    }
+    return d;
+}
+
+// The lane's leaf of staged segment j: its node c at depth d, and the mask of
+// the group's lanes that hold a leaf of their own.
+template <int L>
+__device__ __forceinline__ uint64_t decas_group(const float (&stage)[9][kWave], int j, int maxd,
+                                                float tol, Cub& c, int& d) {
+    const int lane = threadIdx.x & (kWave - 1), i = lane & (L - 1);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        c.x[k] = stage[k][j];
+        c.y[k] = stage[4 + k][j];
+    }
+    d = decas_slot(c, maxd, tol, (uint32_t)i);
+    const bool first = i < (1 << maxd) && (i & ((1 << (maxd - d)) - 1)) == 0;
+    const uint64_t m = __ballot(first) >> (lane & ~(L - 1));
+    return L == kWave ? m : m & ((1ull << (L & (kWave - 1))) - 1);
+}
+
+template <int L>
+__global__ __launch_bounds__(kWave * kFlattenWaves) void k_decas_project(
+    const float* __restrict__ cubics_norm, const int32_t* __restrict__ seg_offsets, int P,
+    const float* __restrict__ aa_widths, const float* __restrict__ stroke_widths, int nseg,
+    int img_h, int img_w, int block_x, int block_y, float aabb_pad, int aniso, int maxd, float tol,
+    float* __restrict__ cubics_px, int32_t* __restrict__ seg_tile_ranges,
+    uint32_t* __restrict__ leaf_counts, int32_t* __restrict__ status) {
+    constexpr int G = kWave / L, kSegs = decas_segs(L);
+    __shared__ float stage[9][kWave];
+    __shared__ int32_t bounds[kWave];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        status[0] = 0;
+        status[1] = 0;
+        status[2] = seg_offsets[0];
+        status[3] = seg_offsets[P];
+    }
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t base = (int64_t)blockIdx.x * kSegs;
+    const int nw = (int)min((int64_t)kSegs, (int64_t)nseg - base);
+    const int p = w == 0 ? wave_owner(seg_offsets, P, (int)base, bounds) : 0;
+    if (w == 0 && lane < nw) {
+        const int s = (int)base + lane;
+        const float wd = fmaxf(aa_widths[p], kWidthMin);
+        const float support = fmaxf(0.0f, wd * 3.0f);
+        const float half_sw = stroke_widths ? fmaxf(0.0f, stroke_widths[p]) * 0.5f : 0.0f;
+        const int tbx = (img_w + block_x - 1) / block_x, tby = (img_h + block_y - 1) / block_y;
+        const SegProj r = project_segment(cubics_norm + (size_t)s * 8, 0.5f * (float)img_w,
+                                          0.5f * (float)img_h, half_sw, support, aabb_pad, aniso,
+                                          tbx, tby, (float)block_x, (float)block_y);
+        float4* cp = reinterpret_cast<float4*>(cubics_px + (size_t)s * 8);
+        cp[0] = make_float4(r.px[0], r.py[0], r.px[1], r.py[1]);
+        cp[1] = make_float4(r.px[2], r.py[2], r.px[3], r.py[3]);
+        reinterpret_cast<int4*>(seg_tile_ranges)[s] = make_int4(r.tx0, r.ty0, r.tx1, r.ty1);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            stage[k][lane] = r.px[k];
+            stage[4 + k][lane] = r.py[k];
+        }
+    }
+    __syncthreads();
+    for (int q = w * G; q < nw; q += kFlattenWaves * G) {
+        const int j = q + lane / L;
+        Cub c;
+        int d;
+        const uint64_t m = decas_group<L>(stage, min(j, nw - 1), maxd, tol, c, d);
+        if (j < nw && (lane & (L - 1)) == 0) leaf_counts[base + j] = (uint32_t)__popcll(m);
+    }
+}
+
+// The leaves' edges, aux and segment records (outputs of k_decas_emit).  With
+// `offsets` null the workgroup makes its segments' edge offsets itself, from
+// the counts of all earlier segments, and writes them to seg_edge_offsets
+// (one launch and its single-workgroup scan less; the caller does so up to
+// kDecasOwnScan segments, where reading the counts costs no more).
+constexpr int kDecasOwnScan = 32768;
+
+template <int L>
+__global__ __launch_bounds__(kWave * kFlattenWaves) void k_decas_emit_wave(
+    const float* __restrict__ cubics_px, const int32_t* __restrict__ seg_offsets, int P,
+    const float* __restrict__ aa_widths, const float* __restrict__ stroke_widths,
+    const float* __restrict__ opacities, int mode, int nseg, int maxd, float tol,
+    const uint32_t* __restrict__ leaf_counts, const int32_t* __restrict__ offsets,
+    int32_t* __restrict__ seg_edge_offsets, EdgeRec* __restrict__ edges,
+    EdgeCull* __restrict__ culls, EdgeAux* __restrict__ aux, SegRec* __restrict__ seg_recs) {
+    constexpr int G = kWave / L, kSegs = decas_segs(L);
+    __shared__ float stage[9][kWave];
+    __shared__ int32_t bounds[kWave], start[kWave];
+    __shared__ uint32_t before_w[kFlattenWaves];
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t base = (int64_t)blockIdx.x * kSegs;
+    const int nw = (int)min((int64_t)kSegs, (int64_t)nseg - base);
+    if (!offsets) {
+        uint32_t sum = 0;
+#pragma unroll 4
+        for (int i = (int)threadIdx.x; i < (int)base; i += kWave * kFlattenWaves)
+            sum += leaf_counts[i];
+        sum = wave_incl_scan_u32(sum);
+        if (lane == kWave - 1) before_w[w] = sum;
+    }
+    const int p = w == 0 ? wave_owner(seg_offsets, P, (int)base, bounds) : 0;
+    if (w == 0 && lane < nw) {
+        const float4* c = reinterpret_cast<const float4*>(cubics_px + (size_t)(base + lane) * 8);
+        const float4 a = c[0], b = c[1];
+        stage[0][lane] = a.x; stage[4][lane] = a.y; stage[1][lane] = a.z; stage[5][lane] = a.w;
+        stage[2][lane] = b.x; stage[6][lane] = b.y; stage[3][lane] = b.z; stage[7][lane] = b.w;
+        stage[8][lane] = prim_params(mode, aa_widths[p], opacities[p], stroke_widths, p).cull_d;
+    }
+    __syncthreads();
+    if (w == 0) {
+        if (offsets) {
+            start[lane] = lane < nw ? offsets[base + lane] : 0;
+        } else {
+            uint32_t e0 = 0;
+#pragma unroll
+            for (int q = 0; q < kFlattenWaves; ++q) e0 += before_w[q];
+            const uint32_t n = lane < nw ? leaf_counts[base + lane] : 0u;
+            const uint32_t incl = wave_incl_scan_u32(n);
+            const int32_t mine = (int32_t)(e0 + incl - n);
+            start[lane] = mine;
+            if (lane < nw) seg_edge_offsets[base + lane] = mine;
+            if (lane < nw && base + lane == nseg - 1) seg_edge_offsets[nseg] = mine + (int32_t)n;
+        }
+    }
+    __syncthreads();
+    const int i = lane & (L - 1);
+    for (int q = w * G; q < nw; q += kFlattenWaves * G) {
+        const int j = q + lane / L;
+        const bool ok = j < nw;
+        const int jc = min(j, nw - 1);
+        const int s = (int)base + jc;
+        Cub c;
+        int d;
+        const uint64_t m = decas_group<L>(stage, jc, maxd, tol, c, d);
+        if (ok && ((m >> i) & 1u)) {
+            const int e = start[jc] + (int)__popcll(m & ((1ull << i) - 1));
+            write_edge(c.x[0], c.y[0], c.x[3], c.y[3], stage[8][jc], edges + e, culls + e);
+            const float2 t = leaf_interval(d, (uint32_t)i >> (maxd - d));
+            *reinterpret_cast<int4*>(aux + e) =
+                make_int4(s, __builtin_bit_cast(int, t.x), __builtin_bit_cast(int, t.y), 0);
+        }
+        // The vertices' box: the root's first point and every leaf's last.
+        VBox box = vbox_empty();
+        vbox_add(box, stage[0][jc], stage[4][jc]);
+        vbox_add(box, c.x[3], c.y[3]);
+#pragma unroll
+        for (int off = L / 2; off >= 1; off >>= 1) {
+            box.x0 = fminf(box.x0, __shfl_xor(box.x0, off, L));
+            box.x1 = fmaxf(box.x1, __shfl_xor(box.x1, off, L));
+            box.y0 = fminf(box.y0, __shfl_xor(box.y0, off, L));
+            box.y1 = fmaxf(box.y1, __shfl_xor(box.y1, off, L));
+        }
+        if (ok && i == 0) seg_recs[s] = seg_record(box, stage[8][jc]);
+    }
+}
+
 // Adaptive flattening, second pass (cubic_splatting.py:1729-1832): the leaves
 // of segment s, left to right, as edges seg_edge_offsets[s] + i (chord P0 ->
 // P3 of leaf i) with their records, the (segment, t0, t1) aux records and the
@@ -2228,6 +2407,7 @@ static int bin_prepare(const float* cubics_norm, const int32_t* seg_offsets, con
         return CS_ERR_ARGS;
     }
     const int tbx = (img_w + block_x - 1) / block_x, tby = (img_h + block_y - 1) / block_y;
+    const bool lane_decas = adaptive && nseg > 0 && maxd <= kDecasLaneDepth;
     if (!adaptive && nseg > 0 && samples <= kWave) {
         // One lane per sample point; the kernel also sets the status words.
         const int lanes = samples <= 2 ? 2 : 1 << ceil_log2(samples);
@@ -2249,11 +2429,43 @@ static int bin_prepare(const float* cubics_norm, const int32_t* seg_offsets, con
             default: CS_FLATTEN_LANES(64); break;
         }
 #undef CS_FLATTEN_LANES
-    } else {
+    } else if (!lane_decas) {
         hipLaunchKernelGGL(k_status_init, dim3(1), dim3(1), 0, stream, seg_offsets, nprim,
                            status);
     }
-    if (nseg > 0 && (adaptive || samples > kWave))
+    if (lane_decas) {
+        const int lanes = maxd < 1 ? 2 : 1 << maxd;
+        const dim3 grid((unsigned)blocks_for(nseg, decas_segs(lanes))),
+            block(kWave * kFlattenWaves);
+        const bool scan = nseg > kDecasOwnScan;
+        int rc = CS_OK;
+#define CS_DECAS_LANES(Lv)                                                                     \
+    hipLaunchKernelGGL(k_decas_project<Lv>, grid, block, 0, stream, cubics_norm, seg_offsets,  \
+                       nprim, aa_widths, stroke_widths, nseg, img_h, img_w, block_x, block_y,  \
+                       aabb_pad, aniso, maxd, kDecasTolPx, cubics_px, seg_tile_ranges,         \
+                       leaf_counts, status);                                                   \
+    if (scan)                                                                                  \
+        rc = cs_scan_exclusive_u32(leaf_counts, reinterpret_cast<uint32_t*>(seg_edge_offsets), \
+                                   nseg, scan_temp, seg_edge_offsets + nseg, stream);          \
+    if (!rc)                                                                                   \
+    hipLaunchKernelGGL(k_decas_emit_wave<Lv>, grid, block, 0, stream, cubics_px, seg_offsets,  \
+                       nprim, aa_widths, stroke_widths, opacities, mode, nseg, maxd,           \
+                       kDecasTolPx, leaf_counts, scan ? seg_edge_offsets : nullptr,            \
+                       seg_edge_offsets, reinterpret_cast<EdgeRec*>(edges),                    \
+                       reinterpret_cast<EdgeCull*>(edge_culls),                                \
+                       reinterpret_cast<EdgeAux*>(edge_aux),                                   \
+                       reinterpret_cast<SegRec*>(seg_recs))
+        switch (lanes) {
+            case 2: CS_DECAS_LANES(2); break;
+            case 4: CS_DECAS_LANES(4); break;
+            case 8: CS_DECAS_LANES(8); break;
+            case 16: CS_DECAS_LANES(16); break;
+            case 32: CS_DECAS_LANES(32); break;
+            default: CS_DECAS_LANES(64); break;
+        }
+#undef CS_DECAS_LANES
+        if (rc) return rc;
+    } else if (nseg > 0 && (adaptive || samples > kWave))
         hipLaunchKernelGGL(k_project_flatten, dim3(blocks_for(nseg, 256)), dim3(256), 0, stream,
                            cubics_norm, seg_offsets, nprim, aa_widths, stroke_widths, opacities,
                            mode, nseg, img_h, img_w, block_x, block_y, aabb_pad, aniso, samples,
@@ -2261,7 +2473,7 @@ static int bin_prepare(const float* cubics_norm, const int32_t* seg_offsets, con
                            reinterpret_cast<EdgeRec*>(edges),
                            reinterpret_cast<EdgeCull*>(edge_culls), maxd, kDecasTolPx,
                            adaptive ? leaf_counts : nullptr);
-    if (adaptive) {
+    if (adaptive && !lane_decas) {
         int rc = cs_scan_exclusive_u32(leaf_counts, reinterpret_cast<uint32_t*>(seg_edge_offsets),
                                        nseg, scan_temp, seg_edge_offsets + nseg, stream);
         if (rc) return rc;

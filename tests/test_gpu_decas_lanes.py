@@ -1,0 +1,67 @@
+"""Adaptive flattening with a group of lanes per segment: every depth the lane
+groups take (S = 2 ... 65) and the first the per-thread walk takes (66),
+degenerate and far segments, a last workgroup that is not full, and more
+segments than a workgroup sums the counts of.  Edges, CSR and aux records bit
+for bit against the oracle, and cull and segment records against the per-vertex
+ones."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import hip_bin, oracle_forward
+from repo_amd import synth
+
+DC = "de_casteljau"
+
+
+def _scene(S, P=70, nseg=3):
+    sc = synth.small_scene(S, P=P, nseg=nseg, h=160, w=200, S=S, rmin=0.5, rmax=250.0)
+    c = sc.cubics_norm
+    c[5] = c[5, :1]                      # a point
+    c[7, 1:] = c[7, :1] + 1e-7           # shorter than the chord floor
+    c[9, 3] = c[9, 0]                    # a loop: no chord
+    c[11, 1] = 40.0                      # far control point
+    c[13, 2] = float("nan")
+    return sc
+
+
+def _check(sc):
+    b, _ = hip_bin(sc, flatten_method=DC)
+    fw = oracle_forward(sc, rows=(0, 1), flatten_method=DC)
+    seo = b.seg_edge_offsets.cpu().numpy()
+    np.testing.assert_array_equal(seo, fw["segment_edge_offsets"])
+    E = int(seo[-1])
+    bits = lambda a: np.ascontiguousarray(a).view(np.int32)  # noqa: E731
+    edges = b.edges[:E].cpu().numpy()
+    np.testing.assert_array_equal(bits(edges[:, :4].reshape(-1, 2, 2)), bits(fw["edges"]))
+    aux = b.edge_aux[:E].cpu().numpy()
+    np.testing.assert_array_equal(aux[:, 0], np.repeat(np.arange(b.nseg), np.diff(seo)))
+    np.testing.assert_array_equal(bits(aux[:, 1].view(np.float32)), bits(fw["edge_t_starts"]))
+    np.testing.assert_array_equal(bits(aux[:, 2].view(np.float32)), bits(fw["edge_t_ends"]))
+    # A segment's near-row union covers its edges' (nothing is culled that an
+    # edge needs): [lo, lo + span - 7] in the records, packed per edge.
+    culls = b.edge_culls[:E].cpu().numpy()
+    recs = b.seg_recs.cpu().numpy()
+    lo, span = (culls[:, 0] << 16) >> 16, culls[:, 0] >> 16
+    seg = aux[:, 0]
+    ok = np.isfinite(edges[:, :4]).all(1)
+    r_lo, r_hi = recs[seg, 0], recs[seg, 0] + recs[seg, 1] - 7
+    # (Packed ranges are clamped to [-2, 16400], which no image row passes.)
+    assert (lo[ok] >= np.clip(r_lo[ok], -2, 16400)).all()
+    assert (lo[ok] + span[ok] - 7 <= np.clip(r_hi[ok], -2, 16400)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [2, 3, 4, 5, 8, 9, 12, 17, 24, 33, 34, 64, 65, 66])
+def test_every_depth(S):
+    print(f"[decas lanes] S={S}", flush=True)
+    _check(_scene(S))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("P", [1, 10923, 10924])
+def test_segment_counts(P):
+    """3, 32769 (the scan's first) and 32772 segments."""
+    print(f"[decas lanes] P={P}", flush=True)
+    sc = synth.small_scene(4, P=P, nseg=3, h=64, w=64, S=6, rmax=12.0)
+    _check(sc)
