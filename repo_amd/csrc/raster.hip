@@ -872,8 +872,10 @@ __global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(
                 for (int p = 0; p < kPix; ++p) cov[p] = 1.0f;
             } else {
                 Geom G[kPix];
-                prim_geometry<MODE, 1, COUNT, MODE == 0>(pr, W, culls, edges, L.px, L.py, cm0, G,
-                                                         n, npix);
+                // (The best edge is only logged: without a log the edges are
+                // visited in any order and only the minimum is kept.)
+                prim_geometry<MODE, LOG ? 1 : 0, COUNT, MODE == 0>(pr, W, culls, edges, L.px, L.py,
+                                                                   cm0, G, n, npix);
                 bool ex[kPix], ins[kPix];
 #pragma unroll
                 for (int p = 0; p < kPix; ++p) {
@@ -909,10 +911,12 @@ __global__ __launch_bounds__(kRasterThreads) __attribute__((amdgpu_waves_per_eu(
                         4 * d0, (int)pack_d2_inside(G[0].min_d2, ins[0]));
                     const uint32_t b = (uint32_t)__builtin_amdgcn_ds_permute(
                         4 * d1, (int)pack_d2_inside(G[1].min_d2, ins[1]));
-                    const int ba = __builtin_amdgcn_ds_permute(4 * d0, G[0].best);
-                    const int bb = __builtin_amdgcn_ds_permute(4 * d1, G[1].best);
                     const uint32_t v = lane < n0 ? a : b;
-                    best_g = lane < n0 ? ba : bb;
+                    if constexpr (LOG) {
+                        const int ba = __builtin_amdgcn_ds_permute(4 * d0, G[0].best);
+                        const int bb = __builtin_amdgcn_ds_permute(4 * d1, G[1].best);
+                        best_g = lane < n0 ? ba : bb;
+                    }
                     if (lane < nx)
                         cov_g = exact_coverage<MODE>(
                             pr, __builtin_bit_cast(float, v & 0x7fffffffu), (v >> 31) != 0);
