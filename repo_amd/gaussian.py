@@ -18,17 +18,18 @@ from typing import Optional
 import torch
 
 from . import _native as N
-from .splat import _give_pinned, _layout, _take_pinned
+from .splat import _dense, _give_pinned, _layout, _take_pinned
 
 GS_RECORD_FLOATS = N.GS_RECORD_BYTES // 4
 
 
+# (Only the tensors' addresses are taken.)
 def _f32(t: torch.Tensor) -> torch.Tensor:
-    return t.detach().to(torch.float32).contiguous()
+    return _dense(t, torch.float32)
 
 
 def _i32(t: torch.Tensor) -> torch.Tensor:
-    return t.detach().to(torch.int32).contiguous()
+    return _dense(t, torch.int32)
 
 
 def tile_bounds(img_h: int, img_w: int, block_x: int, block_y: int):
@@ -125,6 +126,10 @@ class GsBinned:
         self.gaussian_ids_sorted: Optional[torch.Tensor] = None
         self.num_intersects = 0
         self.grad_accum_clean = True
+        # Set while the intersection count has not been read (bin_gaussians
+        # with a capacity hint): (pinned status buffer, capacity of the ids,
+        # cs_bin_finish into a new buffer); resolve_gaussians() settles it.
+        self.pending = None
 
     def ptr(self, name: str) -> int:
         return self._base + self._table[name][0]
@@ -144,12 +149,42 @@ class GsBinned:
         return v
 
 
+def _read_count(pinned) -> int:
+    N.hip_check(N.hip().hipEventSynchronize(pinned[1]), "hipEventSynchronize")
+    I = int(pinned[0][0])
+    _give_pinned(pinned)
+    if I < 0:
+        raise RuntimeError(f"intersection count overflowed int32 ({I})")
+    if I < 1:
+        raise RuntimeError("No intersections generated; increase num_points or radii")
+    return I
+
+
+def resolve_gaussians(b: GsBinned) -> bool:
+    """Reads the intersection count of a bin_gaussians call with a capacity
+    hint.  Returns True when the lists did not fit and were rebuilt at full
+    size (outputs computed from the first build must be computed again)."""
+    if b.pending is None:
+        return False
+    pinned, capacity, finish = b.pending
+    b.pending = None
+    I = b.num_intersects = _read_count(pinned)
+    if I <= capacity:
+        b.gaussian_ids_sorted = b.gaussian_ids_sorted[:I]
+        return False
+    b.gaussian_ids_sorted = finish(I, None)
+    return True
+
+
 def bin_gaussians(xys, conics, radii, depths, img_h: int, img_w: int, block_x: int,
-                  block_y: int) -> GsBinned:
+                  block_y: int, capacity_hint: Optional[int] = None) -> GsBinned:
     """gaussian_ids_sorted and tile_bins of the reference's map + stable sort
     + tile-bin pass (tilelang_renderer.py:224-269), with the backward's
     gradient accumulators cleared in the same launches.  Raises the
-    reference's RuntimeError when there are no intersections."""
+    reference's RuntimeError when there are no intersections.  With a
+    capacity_hint the lists go into a buffer of that many entries without
+    waiting for the count, and the result is pending until
+    resolve_gaussians()."""
     _check_block(block_x, block_y)
     xy, q, rad, d = _f32(xys), _f32(conics), _i32(radii).view(-1), _f32(depths).view(-1)
     n = int(xy.shape[0])
@@ -173,26 +208,29 @@ def bin_gaussians(xys, conics, radii, depths, img_h: int, img_w: int, block_x: i
                q_("keys_alt"), q_("vals_alt"), q_("radix_counts"), q_("scan_temp"),
                q_("rank_tile_ranges"), q_("tile_count"), q_("tile_scratch"), q_("status"), st)
     pinned = _take_pinned(dev.index if dev.index is not None else torch.cuda.current_device())
-    status_host, event = pinned[0], pinned[1]
+    status_host, event, status_dev = pinned[0], pinned[1], pinned[3]
     hip = N.hip()
+
+    def finish(capacity, status_out):
+        ids = torch.empty((capacity,), dtype=torch.int32, device=dev)
+        with N.prof("gs.fwd.bin_finish"):
+            N.call("cs_bin_finish", q_("order"), q_("rank_tile_ranges"), n, q_("status"),
+                   capacity, int(img_h), int(img_w), int(block_x), int(block_y),
+                   q_("tile_count"), q_("tile_scratch"), N.ptr(ids), q_("tile_bins"),
+                   q_("grad_accum"), 9 * n, status_out, st)
+        return ids
+
+    if capacity_hint is not None and status_dev is not None:
+        capacity = max(1, int(capacity_hint))
+        b.gaussian_ids_sorted = finish(capacity, status_dev)
+        N.hip_check(hip.hipEventRecord(event, st), "hipEventRecord")
+        b.pending = (pinned, capacity, finish)
+        return b
     N.hip_check(hip.hipMemcpyAsync(status_host.data_ptr(), q_("status"), 16,
                                    N.HIP_MEMCPY_DEVICE_TO_HOST, st), "hipMemcpyAsync")
     N.hip_check(hip.hipEventRecord(event, st), "hipEventRecord")
-    N.hip_check(hip.hipEventSynchronize(event), "hipEventSynchronize")
-    I = int(status_host[0])
-    _give_pinned(pinned)
-    if I < 0:
-        raise RuntimeError(f"intersection count overflowed int32 ({I})")
-    if I < 1:
-        raise RuntimeError("No intersections generated; increase num_points or radii")
-    ids = torch.empty((I,), dtype=torch.int32, device=dev)
-    with N.prof("gs.fwd.bin_finish"):
-        N.call("cs_bin_finish", q_("order"), q_("rank_tile_ranges"), n, q_("status"), I,
-               int(img_h), int(img_w), int(block_x), int(block_y), q_("tile_count"),
-               q_("tile_scratch"), N.ptr(ids), q_("tile_bins"),
-               q_("grad_accum"), 9 * n, None, st)
-    b.gaussian_ids_sorted = ids
-    b.num_intersects = I
+    I = b.num_intersects = _read_count(pinned)
+    b.gaussian_ids_sorted = finish(I, None)
     return b
 
 

@@ -126,14 +126,16 @@ class _TileLangMSEFn(torch.autograd.Function):
         need_x, need_y = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         if not (need_x or need_y):
             return None, None, None, None, None
-        g = grad_output.detach().to(torch.float32).contiguous()
+        g = (grad_output if grad_output.dtype is torch.float32 and grad_output.is_contiguous()
+             else grad_output.detach().to(torch.float32).contiguous())
         gx = torch.empty_like(x) if need_x else None
         gy = torch.empty_like(y) if need_y else None
         with N.prof("loss.mse_bwd"):
             N.call("cs_mse_backward", N.ptr(x), N.ptr(y), x.numel(), N.ptr(g), N.ptr(gx), N.ptr(gy),
                    N.stream(x.device))
         if gx is not None:
-            gx = gx.view(ctx.shape).to(ctx.x_dtype)
+            gx = gx.view(ctx.shape)
+            gx = gx if ctx.x_dtype is torch.float32 else gx.to(ctx.x_dtype)
         if gy is not None:
             gy = gy.view(ctx.shape).to(ctx.y_dtype)
         return gx, gy, None, None, None

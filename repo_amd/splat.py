@@ -70,6 +70,19 @@ def _f32(t: torch.Tensor) -> torch.Tensor:
     return t.detach().to(torch.float32).contiguous()
 
 
+def _flat(t: torch.Tensor) -> torch.Tensor:
+    """t.reshape(-1), without the call for a 1-D tensor."""
+    return t if t.dim() == 1 else t.reshape(-1)
+
+
+def _dense(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """t itself when it is contiguous and of that dtype (for its address: no
+    detached alias is made), else a contiguous copy of that dtype."""
+    if t.dtype is dtype and t.is_contiguous():
+        return t
+    return t.detach().to(dtype).contiguous()
+
+
 def image_grad_layout(v: torch.Tensor):
     """(tensor, planar) for an upstream image gradient of shape [H, W, 3]:
     the gradient itself when it is float32 and [H, W, 3]-contiguous
@@ -217,6 +230,9 @@ class Binned:
         self.log_key = None
         self.log_units = 0
         self.grad_accum_clean = True
+        self.grad_n = int(table["grad_accum"][2][0])
+        # The last forward's final_Ts, final_idx and log index, one buffer.
+        self.aux: Optional[torch.Tensor] = None
         # The last 4 words of grad_accum (zeroed with it by the binning) count
         # the raster log's shared blocks of the first forward after a binning;
         # log_ctr = (address, first shared unit) when a forward used them.
@@ -228,6 +244,14 @@ class Binned:
 
     def ptr(self, name: str) -> int:
         return self._base + self._table[name][0]
+
+    def grad_accum_part(self, first: int, shape) -> torch.Tensor:
+        """The contiguous `shape` elements of grad_accum from `first` on."""
+        f = self._views.get("")
+        if f is None:
+            f = self._views[""] = self.arena.view(torch.float32)
+        stride = (shape[1], 1) if len(shape) == 2 else (1,)
+        return f.as_strided(shape, stride, self._table["grad_accum"][0] // 4 + first)
 
     def __getattr__(self, name):
         table = self.__dict__.get("_table")
@@ -602,6 +626,26 @@ def rasterize_forward(b: Binned, background: torch.Tensor, eval_counts=None, log
     size on this stream (if any); every ORDER_EVERY-th forward records its
     wave durations and makes a new order from them, which its backward
     (b.tile_order) and the following forwards take."""
+    out = _forward_launch(b, background, eval_counts, log, log_pool_bytes_override)
+    final_T, final_idx = forward_state(b)
+    return out, final_T, final_idx
+
+
+def forward_state(b: Binned):
+    """(final_Ts [H, W], final_idx [H, W]) of b's last forward."""
+    H, W = b.img_h, b.img_w
+    return (b.aux[:H * W].view(torch.float32).view(H, W), b.aux[H * W:2 * H * W].view(H, W))
+
+
+# Launches over at most this many sub-blocks take no tile order: all of their
+# workgroups are resident at once (512 blocks of eight waves, two or more per
+# CU), so it does not matter in which order they start.
+ORDER_MIN_SUB_BLOCKS = 256
+
+
+def _forward_launch(b: Binned, background, eval_counts=None, log=True,
+                    log_pool_bytes_override=None):
+    """rasterize_forward without views of T and the index, which stay in b.aux."""
     dev = b.device
     H, W = b.img_h, b.img_w
     out = torch.empty((H, W, 3), dtype=torch.float32, device=dev)
@@ -613,9 +657,8 @@ def rasterize_forward(b: Binned, background: torch.Tensor, eval_counts=None, log
     cap = max(int(b.primitive_ids_sorted.numel()), 1)
     # final_Ts, final_idx and the log's entry index share one allocation.
     n_index = wpt * cap if log else 0
-    aux = torch.empty((2 * H * W + n_index,), dtype=torch.int32, device=dev)
-    final_T = aux[:H * W].view(torch.float32).view(H, W)
-    final_idx = aux[H * W:2 * H * W].view(H, W)
+    aux = b.aux = torch.empty((2 * H * W + n_index,), dtype=torch.int32, device=dev)
+    base = aux.data_ptr()
     st = N.stream(dev)
     if log:
         key = b.log_key if b.log_key is not None else (
@@ -626,18 +669,18 @@ def rasterize_forward(b: Binned, background: torch.Tensor, eval_counts=None, log
             units, pool_bytes = 0, max(16, int(log_pool_bytes_override) // 16 * 16)
         b.log_index = aux[2 * H * W:]
         b.log_pool = torch.empty((pool_bytes,), dtype=torch.uint8, device=dev)
+        pool_p = b.log_pool.data_ptr()
         b.log_units = units
         # The first forward after a binning counts its shared blocks in the
         # gradient buffer's zeroed counter word (no set-up launch); a repeated
         # forward lets the library set up the pool's own counter.
         ctr = None
         first_shared = 1 + wpt * cap * units
-        if b.log_ctr_clean and b.grad_accum is not None:
-            ga = b.grad_accum
-            ctr = ga.data_ptr() + 4 * (ga.numel() - _LOG_COUNTER_ELEMS)
+        if b.log_ctr_clean:
+            ctr = b.ptr("grad_accum") + 4 * (b.grad_n - _LOG_COUNTER_ELEMS)
             b.log_ctr_clean = False
         b.log_ctr = None if ctr is None else (ctr, first_shared)
-        log_args = (cap, b.log_index.data_ptr(), b.log_pool.data_ptr(), pool_bytes, units, ctr)
+        log_args = (cap, base + 8 * H * W, pool_p, pool_bytes, units, ctr)
     else:
         b.log_index = b.log_pool = None
         b.log_ctr = None
@@ -645,10 +688,12 @@ def rasterize_forward(b: Binned, background: torch.Tensor, eval_counts=None, log
     # The tile order is kept apart: the next forward reads it after this
     # forward's buffers are gone.
     okey = (dev.index, st, nsub)
-    prev = _TILE_ORDERS.get(okey)
-    age = _ORDER_AGE.get(okey, 0) + 1
-    remake = prev is None or age >= ORDER_EVERY or eval_counts is not None
-    base = aux.data_ptr()
+    if nsub <= ORDER_MIN_SUB_BLOCKS and eval_counts is None:
+        prev, age, remake = None, 0, False
+    else:
+        prev = _TILE_ORDERS.get(okey)
+        age = _ORDER_AGE.get(okey, 0) + 1
+        remake = prev is None or age >= ORDER_EVERY or eval_counts is not None
     args = (b.mode, N.ptr(b.primitive_ids_sorted), b.ptr("tile_bins"), b.ptr("edges"),
             b.ptr("edge_culls"), b.ptr("prim_recs"), N.ptr(background), H, W, b.block_x,
             b.block_y, b.edges_per_segment, out.data_ptr(), 0, planes.data_ptr(), base,
@@ -667,12 +712,13 @@ def rasterize_forward(b: Binned, background: torch.Tensor, eval_counts=None, log
         if b.log_ctr is not None:
             _read_log_use_later(key, dix, b.log_ctr[0], 0, units, first_shared, pool_bytes, st)
         else:
-            _read_log_use_later(key, dix, b.log_pool.data_ptr(), first_shared, units,
+            _read_log_use_later(key, dix, pool_p, first_shared, units,
                                 first_shared, pool_bytes, st)
     if not remake:
         b.tile_order = prev
-        _ORDER_AGE[okey] = age
-        return out, final_T, final_idx
+        if prev is not None:
+            _ORDER_AGE[okey] = age
+        return out
     order = torch.empty((int(N.lib().cs_raster_tile_order_elems(nsub)),), dtype=torch.int32,
                         device=dev)
     last, spare = _TILE_COSTS.get(okey, (None, None))
@@ -692,7 +738,7 @@ def rasterize_forward(b: Binned, background: torch.Tensor, eval_counts=None, log
         _TILE_COSTS.pop(old, None)
     _TILE_ORDERS[okey] = order
     _ORDER_AGE[okey] = 0
-    return out, final_T, final_idx
+    return out
 
 
 def _rasterize_forward_any(b: Binned, background, planes, out, eval_counts):
@@ -702,18 +748,17 @@ def _rasterize_forward_any(b: Binned, background, planes, out, eval_counts):
         raise ValueError("evaluation counts are measured on 16x16 sub-block tiles only")
     dev = b.device
     H, W = b.img_h, b.img_w
-    aux = torch.empty((2 * H * W,), dtype=torch.int32, device=dev)
-    final_T = aux[:H * W].view(torch.float32).view(H, W)
-    final_idx = aux[H * W:].view(H, W)
+    b.aux = torch.empty((2 * H * W,), dtype=torch.int32, device=dev)
+    base = b.aux.data_ptr()
     b.log_index = b.log_pool = None
     b.log_ctr = None
     b.tile_order = None
     with N.prof("cubic.fwd.rast"):
         N.call("cs_rasterize_forward_any_tile", b.mode, N.ptr(b.primitive_ids_sorted),
                b.ptr("tile_bins"), b.ptr("edges"), b.ptr("prim_recs"), N.ptr(background), H, W,
-               b.block_x, b.block_y, out.data_ptr(), 0, planes.data_ptr(), final_T.data_ptr(),
-               final_idx.data_ptr(), N.stream(dev))
-    return out, final_T, final_idx
+               b.block_x, b.block_y, out.data_ptr(), 0, planes.data_ptr(), base,
+               base + 4 * H * W, N.stream(dev))
+    return out
 
 
 def _rasterize_backward_any(b: Binned, background, final_T, final_idx, v_output, planar, v_px,
@@ -829,36 +874,47 @@ def rasterize_backward_finalized(b: Binned, background, final_T, final_idx, v_ou
     copies' reduction and the epilogue in one launch
     (cs_rasterize_backward_finalized): returns (v_cubics_norm [nseg,4,2],
     v_colors [P,3], v_opacities [P], v_aa_widths [P], v_stroke_widths [P] or
-    None), the values of the two calls.  Uniform flattening and 16 x 16
-    sub-block tiles (the other backward kernels keep the two calls)."""
+    None), the values of the two calls; final_T and final_idx None: those of
+    b's last forward.  Uniform flattening and 16 x 16 sub-block tiles (the
+    other backward kernels keep the two calls)."""
     dev = b.device
-    P = b.nprim
+    P, n_cp = b.nprim, b.nseg * 8
+    stroke = b.mode == MODE_STROKE
+    nv = 6 if stroke else 5
     if b.grad_accum_clean:
-        zeros = b.grad_accum
+        part, px_p = b.grad_accum_part, b.ptr("grad_accum")
         b.grad_accum_clean = False
     else:  # a second backward through the same forward
         zeros = torch.zeros((_grad_accum_elems(b.nseg, P, b.mode),), dtype=torch.float32,
                             device=dev)
-    v_px = zeros[: b.nseg * 8]
-    rest = zeros[b.nseg * 8:]
-    v_colors = rest[: 3 * P].view(P, 3)
-    v_opac = rest[3 * P: 4 * P]
-    v_is2 = rest[4 * P: 5 * P]
-    v_sw = rest[5 * P: 6 * P] if b.mode == MODE_STROKE else None
-    nv = 6 if b.mode == MODE_STROKE else 5
-    out = torch.empty((b.nseg * 8 + P,), dtype=torch.float32, device=dev)
-    v_norm = out[: b.nseg * 8].view(b.nseg, 4, 2)
-    v_aa = out[b.nseg * 8:]
+
+        def part(first, shape):
+            n = shape[0] * (shape[1] if len(shape) == 2 else 1)
+            return zeros[first:first + n].view(shape)
+        px_p = zeros.data_ptr()
+    # v_px, then the per-primitive sums and their copies.
+    v_colors = part(n_cp, (P, 3))
+    v_opac = part(n_cp + 3 * P, (P,))
+    v_sw = part(n_cp + 5 * P, (P,)) if stroke else None
+    prim_p = px_p + 4 * n_cp
+    out = torch.empty((n_cp + P,), dtype=torch.float32, device=dev)
+    v_norm = out[:n_cp].view(b.nseg, 4, 2)
+    v_aa = out[n_cp:]
     v_output, planar = image_grad_layout(v_output)
+    if final_T is None:
+        T_p = b.aux.data_ptr()
+        idx_p = T_p + 4 * b.img_h * b.img_w
+    else:
+        T_p, idx_p = final_T.data_ptr(), final_idx.data_ptr()
     with N.prof("cubic.bwd.rast"):
         N.call("cs_rasterize_backward_finalized", b.mode, N.ptr(b.primitive_ids_sorted),
                b.ptr("tile_bins"), b.ptr("edges"), b.ptr("edge_culls"), b.ptr("prim_recs"),
                N.ptr(background), b.img_h, b.img_w, b.block_x, b.block_y,
-               b.edges_per_segment, N.ptr(final_T), N.ptr(final_idx), N.ptr(b.log_index),
-               N.ptr(b.log_pool), N.ptr(v_output), planar, N.ptr(v_px), N.ptr(v_colors),
-               N.ptr(v_opac), N.ptr(v_is2), N.ptr(v_sw), P, N.ptr(rest[nv * P:]),
-               N.ptr(b.tile_order), b.nseg, N.ptr(widths), N.ptr(v_norm), N.ptr(v_aa),
-               N.stream(dev))
+               b.edges_per_segment, T_p, idx_p, N.ptr(b.log_index),
+               N.ptr(b.log_pool), N.ptr(v_output), planar, px_p, prim_p,
+               prim_p + 12 * P, prim_p + 16 * P, prim_p + 20 * P if stroke else None, P,
+               prim_p + 4 * nv * P, N.ptr(b.tile_order), b.nseg, N.ptr(widths), N.ptr(v_norm),
+               N.ptr(v_aa), N.stream(dev))
     return v_norm, v_colors, v_opac, v_aa, v_sw
 
 
@@ -948,7 +1004,7 @@ def _splat_forward(ctx, mode, cubics_norm, primitive_seg_offsets, colors, opacit
                    process_fn):
     flatten_method_norm = normalize_cubic_flatten_method(flatten_method)
     num_segments = int(cubics_norm.shape[0])
-    offs = _i32(primitive_seg_offsets).view(-1)
+    offs = _flat(_dense(primitive_seg_offsets, torch.int32))
     num_primitives = max(0, int(offs.numel()) - 1)
     dev = cubics_norm.device
     bg = background
@@ -969,7 +1025,7 @@ def _splat_forward(ctx, mode, cubics_norm, primitive_seg_offsets, colors, opacit
                        ("stroke_widths", stroke_widths, 1)):
         if t is None:
             continue
-        n = int(t.shape[0]) if k is None else int(t.reshape(-1).shape[0])
+        n = int(t.shape[0]) if k is None else int(t.numel())
         if n != num_primitives:
             raise ValueError(
                 f"{name} size must match primitive count ({num_primitives}), got {n}"
@@ -977,21 +1033,22 @@ def _splat_forward(ctx, mode, cubics_norm, primitive_seg_offsets, colors, opacit
                 f"colors first dim must match primitive count ({num_primitives}), got {n}")
     # The reference clamps the widths to >= 1e-4 here (cubic_splatting.py:2820);
     # every kernel that reads them applies that clamp itself.
-    widths = _f32(aa_widths).view(-1)
+    widths = _flat(_f32(aa_widths))
     if int(widths.numel()) != num_primitives:
         raise ValueError(
             f"aa_widths size must match primitive count ({num_primitives}), "
             f"got {int(widths.numel())}")
 
     colors_c = _f32(colors)
-    opac_c = _f32(opacities).view(-1)
-    rules_c = _i32(fill_rules).view(-1) if fill_rules is not None else None
-    sw_c = _f32(stroke_widths).view(-1) if stroke_widths is not None else None
+    opac_c = _flat(_f32(opacities))
+    rules_c = _flat(_dense(fill_rules, torch.int32)) if fill_rules is not None else None
+    sw_c = _flat(_f32(stroke_widths)) if stroke_widths is not None else None
     hint_key = (cubics_norm.device.index, mode, num_primitives, num_segments, int(img_h),
                 int(img_w), int(distance_samples), flatten_method_norm, int(block_x),
                 int(block_y))
-    b = bin_primitives(_f32(cubics_norm), offs, colors_c, opac_c, _f32(depths).view(-1),
-                       rules_c, widths, sw_c, int(img_h), int(img_w), int(distance_samples),
+    b = bin_primitives(_dense(cubics_norm, torch.float32), offs, colors_c, opac_c,
+                       _flat(_dense(depths, torch.float32)), rules_c, widths, sw_c, int(img_h),
+                       int(img_w), int(distance_samples),
                        aabb_pad=float(aabb_pad), aniso=bool(aniso_intersects), mode=mode,
                        block_x=int(block_x), block_y=int(block_y),
                        capacity_hint=_CAPACITY_HINTS.get(hint_key),
@@ -1002,9 +1059,9 @@ def _splat_forward(ctx, mode, cubics_norm, primitive_seg_offsets, colors, opacit
     # requires a gradient).
     log = any(ctx.needs_input_grad)
     b.log_key = hint_key
-    out, final_T, final_idx = rasterize_forward(b, bg, log=log)
+    out = _forward_launch(b, bg, log=log)
     if resolve_binned(b):
-        out, final_T, final_idx = rasterize_forward(b, bg, log=log)
+        out = _forward_launch(b, bg, log=log)
     _remember_capacity(hint_key, b.num_intersects)
     if b.num_intersects <= 0:
         ctx.empty = True
@@ -1020,14 +1077,14 @@ def _splat_forward(ctx, mode, cubics_norm, primitive_seg_offsets, colors, opacit
     # made here are plain attributes.
     ctx.save_for_backward(colors_c, opac_c, depths, sw_c)
     ctx.cub_shape = cubics_norm.shape
-    ctx.offs, ctx.widths, ctx.bg, ctx.final_T, ctx.final_idx = offs, widths, bg, final_T, final_idx
+    ctx.offs, ctx.widths, ctx.bg = offs, widths, bg
     return out
 
 
 def _splat_backward(ctx, grad_out_img):
     b: Binned = ctx.binned
     colors, opacities, depths, stroke_widths = ctx.saved_tensors
-    offs, widths, bg, final_T, final_idx = ctx.offs, ctx.widths, ctx.bg, ctx.final_T, ctx.final_idx
+    offs, widths, bg = ctx.offs, ctx.widths, ctx.bg
     process_fn = ctx.process_fn
     curve_contrib_rgb = curve_isect_contrib = None
     if process_fn is not None:
@@ -1047,12 +1104,13 @@ def _splat_backward(ctx, grad_out_img):
     # own last launch.
     if process_fn is None and not b.any_tile and not b.adaptive:
         v_cubics_norm, v_colors, v_opac, v_aa, v_sw = rasterize_backward_finalized(
-            b, bg, final_T, final_idx, grad_out_img, widths)
+            b, bg, None, None, grad_out_img, widths)
         depth_index = 5 if ctx.mode == MODE_STROKE else 4
         v_depths = (torch.zeros_like(depths, dtype=torch.float32)
                     if ctx.needs_input_grad[depth_index] else None)
         return v_cubics_norm.view(ctx.cub_shape), v_colors, v_opac.view_as(opacities), v_sw, \
             v_depths, v_aa
+    final_T, final_idx = forward_state(b)
     v_cubics_px, v_colors, v_opac, v_is2, v_sw = rasterize_backward(
         b, bg, final_T, final_idx, grad_out_img, curve_contrib_rgb=curve_contrib_rgb,
         curve_isect_contrib=curve_isect_contrib)
@@ -1136,7 +1194,8 @@ class _CubicPolylineSplatFunction(torch.autograd.Function):
 def _prim_vector(t, num_primitives, name, device, dtype, default):
     if t is None:
         return torch.full((num_primitives,), default, device=device, dtype=dtype)
-    out = t.to(device=device, dtype=dtype).view(-1)
+    out = t if t.device == device and t.dtype is dtype else t.to(device=device, dtype=dtype)
+    out = out if out.dim() == 1 else out.view(-1)
     if int(out.numel()) == 1 and num_primitives > 1:
         out = out.expand(num_primitives)
     if int(out.numel()) != num_primitives:
@@ -1163,18 +1222,18 @@ def _common_checks(cubics_norm, offs, colors, opacities, depths, num_primitives,
         raise ValueError(
             f"colors first dim must match primitive count ({num_primitives}), "
             f"got {int(colors.shape[0])}")
-    if int(opacities.reshape(-1).shape[0]) != num_primitives:
+    if int(opacities.numel()) != num_primitives:
         raise ValueError(
             f"opacities size must match primitive count ({num_primitives}), "
-            f"got {int(opacities.reshape(-1).shape[0])}")
-    if stroke_widths is not None and int(stroke_widths.reshape(-1).shape[0]) != num_primitives:
+            f"got {int(opacities.numel())}")
+    if stroke_widths is not None and int(stroke_widths.numel()) != num_primitives:
         raise ValueError(
             f"stroke_widths size must match primitive count ({num_primitives}), "
-            f"got {int(stroke_widths.reshape(-1).shape[0])}")
-    if int(depths.reshape(-1).shape[0]) != num_primitives:
+            f"got {int(stroke_widths.numel())}")
+    if int(depths.numel()) != num_primitives:
         raise ValueError(
             f"depths size must match primitive count ({num_primitives}), "
-            f"got {int(depths.reshape(-1).shape[0])}")
+            f"got {int(depths.numel())}")
 
 
 def render_cubic_fill_splat_tilelang(cubics_norm, primitive_seg_offsets, colors, opacities,
@@ -1187,7 +1246,7 @@ def render_cubic_fill_splat_tilelang(cubics_norm, primitive_seg_offsets, colors,
                                      flatten_method=DEFAULT_CUBIC_FLATTEN_METHOD,
                                      process_fn=None):
     """cubic_splatting.py:3128-3229 -> [H, W, 3] image."""
-    offs = _i32(primitive_seg_offsets).view(-1)
+    offs = _flat(_i32(primitive_seg_offsets))
     num_primitives = max(0, int(offs.numel()) - 1)
     if num_primitives <= 0:
         bg = background.to(device=cubics_norm.device, dtype=torch.float32).view(1, 1, 3)
@@ -1201,8 +1260,8 @@ def render_cubic_fill_splat_tilelang(cubics_norm, primitive_seg_offsets, colors,
              .contiguous())
     widths = _aa_widths(aa_widths, num_primitives, dev, aa_width)
     return _CubicFillSplatFunction.apply(
-        cubics_norm, offs.contiguous(), colors.contiguous(), opacities.reshape(-1).contiguous(),
-        depths.reshape(-1).contiguous(), rules, int(img_h), int(img_w),
+        cubics_norm, offs, colors.contiguous(), _flat(opacities).contiguous(),
+        _flat(depths).contiguous(), rules, int(img_h), int(img_w),
         int(block_x), int(block_y), background, int(project_threads), int(map_threads),
         float(aabb_pad), bool(aniso_intersects), widths, int(distance_samples),
         normalize_cubic_flatten_method(flatten_method), process_fn)
@@ -1218,7 +1277,7 @@ def render_cubic_polyline_splat_tilelang(cubics_norm, primitive_seg_offsets, col
                                          flatten_method=DEFAULT_CUBIC_FLATTEN_METHOD,
                                          process_fn=None):
     """cubic_polyline_splatting.py:1341-1432 -> [H, W, 3] image."""
-    offs = _i32(primitive_seg_offsets).view(-1)
+    offs = _flat(_i32(primitive_seg_offsets))
     num_primitives = max(0, int(offs.numel()) - 1)
     if num_primitives <= 0:
         bg = background.to(device=cubics_norm.device, dtype=torch.float32).view(1, 1, 3)
@@ -1227,8 +1286,8 @@ def render_cubic_polyline_splat_tilelang(cubics_norm, primitive_seg_offsets, col
     dev = cubics_norm.device
     widths = _aa_widths(aa_widths, num_primitives, dev, aa_width)
     return _CubicPolylineSplatFunction.apply(
-        cubics_norm, offs.contiguous(), colors.contiguous(), opacities.reshape(-1).contiguous(),
-        stroke_widths.reshape(-1).contiguous(), depths.reshape(-1).contiguous(), int(img_h),
+        cubics_norm, offs, colors.contiguous(), _flat(opacities).contiguous(),
+        _flat(stroke_widths).contiguous(), _flat(depths).contiguous(), int(img_h),
         int(img_w), int(block_x), int(block_y), background, int(project_threads),
         int(map_threads), float(aabb_pad), bool(aniso_intersects), widths,
         int(distance_samples), normalize_cubic_flatten_method(flatten_method), process_fn)
