@@ -1,6 +1,7 @@
 // Forward and backward rasterization of flattened cubic primitives on MI355X.
 //
-// Launch: one 128-thread workgroup per 16x16 tile.  Unlike a block-synchronous
+// Launch: one 128-thread workgroup per 16x16 tile (small images split a tile's
+// list over more waves: split_block).  Unlike a block-synchronous
 // design, each of the two waves owns eight tile rows (128 pixels, two per lane:
 // rows r and r + 4 of one column) and walks the tile's sorted list on its own,
 // so every per-entry scalar step, edge-record load and wave reduction serves
@@ -485,8 +486,8 @@ __device__ __forceinline__ SubBlock sub_block(const TileGrid& tg,
 // that recurrence over the NW entries for itself (about 12 vector operations
 // an entry and pixel, the same operations in the same order as one wave would
 // run, so the results are bit-identical), so no state is handed back.
-// Training step of 64 paths at 128 x 128: forward 135 -> 32 us, backward
-// 73 -> 22 us; the rule is at split_waves.
+// Training step of 64 paths at 128 x 128: forward 135 -> 41 us, backward
+// 73 -> 24 us; the rule is at split_waves.
 __device__ __forceinline__ SubBlock split_block(const TileGrid& tg,
                                                 const int32_t* __restrict__ tile_order) {
     if (tile_order) {

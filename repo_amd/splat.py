@@ -962,7 +962,7 @@ _MAX_HINTS = 64
 def _remember_capacity(key, num_intersects: int) -> None:
     _CAPACITY_HINTS.pop(key, None)
     if len(_CAPACITY_HINTS) >= _MAX_HINTS:
-        _CAPACITY_HINTS.pop(next(iter(_CAPACITY_HINTS)))
+        _CAPACITY_HINTS.pop(next(iter(_CAPACITY_HINTS)), None)
     _CAPACITY_HINTS[key] = intersection_capacity(max(0, num_intersects))
 
 
