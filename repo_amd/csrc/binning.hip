@@ -1685,8 +1685,9 @@ __global__ __launch_bounds__(256) void k_fill_i32(int32_t* __restrict__ a, int n
 //        rectangles against the segment; the hits (primitive id and column
 //        range within the segment) go to one LDS list in rank order, each
 //        wave's after the hits of the slices before it;
-//     2. each wave owns kListTilesPerWave tile columns and reads that list 64
-//        hits at a time: per owned tile a ballot of the hits whose range
+//     2. when the list might not hold another chunk's hits, or after the last
+//        chunk: each wave owns kListTilesPerWave tile columns and reads the
+//        list 64 hits at a time: per owned tile a ballot of the hits whose range
 //        contains it gives, in rank order, the tile's next entries, written
 //        to consecutive slots (mbcnt) of its list.  (Staging them in LDS for
 //        64-wide stores measured slower.)
@@ -1696,6 +1697,13 @@ constexpr int kListTilesPerWave = kSegTiles / kListWaves;
 constexpr int kListChunk = 1024;
 constexpr int kListSlice = kListChunk / kListWaves;
 constexpr int kListSteps = kListSlice / kWave;
+// Hits held in LDS before they are dealt to the tiles.  Small primitives leave
+// few hits in a chunk (about 30 of 1024 for 100000 Gaussians at 1024 x 1024),
+// and dealing them chunk by chunk takes two more barriers a chunk and mostly
+// empty groups of 64: there 41 -> 28 us, and 22 -> 19 us for 16384
+// clustered fills.  (A slab of one chunk keeps the smaller list: 6.3 us against
+// 6.9 for 4096 fills at 2040 x 1356.)
+constexpr int kListHits = 2 * kListChunk;
 constexpr int kMaxSlabs = 64;
 
 // Rank slabs of the list build: nslab slabs of `slab` ranks (a multiple of
@@ -1820,15 +1828,18 @@ __global__ __launch_bounds__(kWave * kListWaves) void k_tile_counts(
     }
 }
 
+// ONE: a slab is a single chunk (no list is carried over).
+template <bool ONE>
 __global__ __launch_bounds__(kWave * kListWaves) void k_tile_scatter(
     const int32_t* __restrict__ order, const int4* __restrict__ rank_rects, int P, int tbx,
     int tby, int nsegcols, int slab, int nslab, const uint32_t* __restrict__ tile_count,
     const uint32_t* __restrict__ seg_scratch, int32_t* __restrict__ prim_ids_sorted,
     int32_t* __restrict__ tile_bins, float* __restrict__ zero_buf, int64_t zero_n,
     const int32_t* __restrict__ total, int64_t capacity, int32_t* __restrict__ status_host) {
-    __shared__ int32_t hit_pid[kListChunk];
-    __shared__ uint32_t hit_cols[kListChunk];
-    __shared__ int hit_n[kListWaves];
+    constexpr int kHeld = ONE ? kListChunk : kListHits;
+    __shared__ int32_t hit_pid[kHeld];
+    __shared__ uint32_t hit_cols[kHeld];
+    __shared__ int hit_n[2][kListWaves];
     __shared__ uint32_t tile_start[kSegTiles];
     // The four status words (final once the counting launch has ended) to the
     // caller's host buffer, which it reads after this launch.
@@ -1855,6 +1866,19 @@ __global__ __launch_bounds__(kWave * kListWaves) void k_tile_scatter(
         }
         return;
     }
+    const int rb = lp.slab * slab, re = min(P, rb + slab);
+    int4 tr[kListSteps];
+    int pid[kListSteps];
+    auto load_chunk = [&](int c0) {
+        const int r0 = c0 + w * kListSlice, r1 = min(r0 + kListSlice, re);
+#pragma unroll
+        for (int k = 0; k < kListSteps; ++k) {
+            const int rr = r0 + k * kWave + lane;
+            tr[k] = rr < r1 ? rank_rects[rr] : make_int4(0, 0, 0, 0);
+            pid[k] = rr < r1 ? order[rr] : 0;
+        }
+    };
+    load_chunk(rb);   // in flight while wave 0 adds the slabs' counts
     if (w == 0) {
         // The tile's count over all slabs, the slabs' counts before this one,
         // and the segment's first slot (summed over the slabs).
@@ -1887,55 +1911,52 @@ __global__ __launch_bounds__(kWave * kListWaves) void k_tile_scatter(
     }
     __syncthreads();
     uint32_t cur[kListTilesPerWave];
-    int nst[kListTilesPerWave];
 #pragma unroll
     for (int k = 0; k < kListTilesPerWave; ++k) {
         cur[k] = tile_start[w * kListTilesPerWave + k];
-        nst[k] = 0;
     }
 
-    const int rb = lp.slab * slab, re = min(P, rb + slab);
-    for (int c0 = rb; c0 < re; c0 += kListChunk) {
-        // 1. Compact the chunk's hits into one list (this wave's loads all
-        //    in flight before the first test).
-        const int r0 = c0 + w * kListSlice;
-        const int r1 = min(r0 + kListSlice, re);
-        int4 tr[kListSteps];
-        int pid[kListSteps];
-#pragma unroll
-        for (int k = 0; k < kListSteps; ++k) {
-            const int rr = r0 + k * kWave + lane;
-            tr[k] = rr < r1 ? rank_rects[rr] : make_int4(0, 0, 0, 0);
-            pid[k] = rr < r1 ? order[rr] : 0;
-        }
+    int nh = 0;   // hits held
+    for (int c0 = rb, odd = 0; c0 < re; c0 += kListChunk, odd ^= 1) {
+        // 1. Append the chunk's hits to the list; the next chunk's loads are
+        //    in flight meanwhile.  (Waves write one chunk's counts while
+        //    others may still read the last one's: two sets.  The barrier also
+        //    stands between a list's readers and its next writers.)
         bool hit[kListSteps];
+        uint32_t cols_w[kListSteps];
+        int pid_w[kListSteps];
         int n_w = 0;
 #pragma unroll
         for (int k = 0; k < kListSteps; ++k) {
-            hit[k] = rect_meets_row(tr[k], ty, sx0, sx1);
+            const int4 q = tr[k];
+            hit[k] = rect_meets_row(q, ty, sx0, sx1);
             n_w += __builtin_popcountll(__ballot(hit[k]));
+            cols_w[k] = (uint32_t)(max(q.x, sx0) - sx0) | ((uint32_t)(min(q.z, sx1) - sx0) << 16);
+            pid_w[k] = pid[k];
         }
-        if (lane == 0) hit_n[w] = n_w;
+        const bool last = ONE || c0 + kListChunk >= re;
+        if (!last) load_chunk(c0 + kListChunk);
+        if (lane == 0) hit_n[odd][w] = n_w;
         __syncthreads();
-        int nh = 0, slot0 = 0;
+        int slot0 = nh;
 #pragma unroll
         for (int v = 0; v < kListWaves; ++v) {
-            const int c = hit_n[v];
+            const int c = hit_n[odd][v];
             slot0 += v < w ? c : 0;
             nh += c;
         }
+        nh = __builtin_amdgcn_readfirstlane(nh);
 #pragma unroll
         for (int k = 0; k < kListSteps; ++k) {
             const uint64_t m = __ballot(hit[k]);
             if (hit[k]) {
-                const int4 q = tr[k];
                 const int slot = slot0 + (int)lanes_below(m);
-                hit_pid[slot] = pid[k];
-                hit_cols[slot] = (uint32_t)(max(q.x, sx0) - sx0) |
-                                 ((uint32_t)(min(q.z, sx1) - sx0) << 16);
+                hit_pid[slot] = pid_w[k];
+                hit_cols[slot] = cols_w[k];
             }
             slot0 += __builtin_popcountll(m);
         }
+        if (!last && nh + kListChunk <= kHeld) continue;
         __syncthreads();
         // 2. The owned tiles' next entries, 64 hits at a time (the next
         //    group's LDS reads in flight).
@@ -1957,7 +1978,8 @@ __global__ __launch_bounds__(kWave * kListWaves) void k_tile_scatter(
                 cur[k] += (uint32_t)__builtin_popcountll(m);
             }
         }
-        __syncthreads();
+        if (ONE) break;
+        nh = 0;
     }
 }
 
@@ -2713,7 +2735,8 @@ extern "C" int cs_bin_finish(const int32_t* order, const int32_t* rank_tile_rang
     const int tbx = (img_w + block_x - 1) / block_x, tby = (img_h + block_y - 1) / block_y;
     const int nsegcols = (tbx + kSegTiles - 1) / kSegTiles;
     const ListSlabs ls = list_slabs(nprim, nsegcols * tby);
-    hipLaunchKernelGGL(k_tile_scatter, dim3(nsegcols * tby * ls.nslab),
+    const auto scatter = ls.slab == kListChunk ? k_tile_scatter<true> : k_tile_scatter<false>;
+    hipLaunchKernelGGL(scatter, dim3(nsegcols * tby * ls.nslab),
                        dim3(kWave * kListWaves), 0, stream, order,
                        reinterpret_cast<const int4*>(rank_tile_ranges), nprim, tbx, tby, nsegcols,
                        ls.slab, ls.nslab, tile_count, tile_scratch, prim_ids_sorted, tile_bins,
