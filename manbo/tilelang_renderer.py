@@ -147,19 +147,24 @@ class GsRenderFunction(torch.autograd.Function):
                 expected_size=gaussian_ids_sorted.shape[0], device=gaussian_ids_sorted.device)
             tile_bins = payload["tile_bins"]
 
-            with _prof(_profile_label(profile_fwd_prefix, "rast")):
-                n = int(xys.shape[0])
-                records = G.pack_records(xys, conics, colors, opacities,
-                                         out=binned.records if n == binned.n else None)
-                out_img, final_Ts, final_idx = G.rasterize_forward(
-                    gaussian_ids_sorted, tile_bins, records, bg, img_h, img_w, block_x, block_y)
-                if G.resolve_gaussians(binned):
+            try:
+                with _prof(_profile_label(profile_fwd_prefix, "rast")):
+                    n = int(xys.shape[0])
+                    records = G.pack_records(xys, conics, colors, opacities,
+                                             out=binned.records if n == binned.n else None)
                     out_img, final_Ts, final_idx = G.rasterize_forward(
-                        binned.gaussian_ids_sorted, tile_bins, records, bg, img_h, img_w, block_x,
+                        gaussian_ids_sorted, tile_bins, records, bg, img_h, img_w, block_x,
                         block_y)
-                if process_fn is None:
-                    gaussian_ids_sorted = binned.gaussian_ids_sorted
-                    S._remember_capacity(hint_key, binned.num_intersects)
+                    if G.resolve_gaussians(binned):
+                        out_img, final_Ts, final_idx = G.rasterize_forward(
+                            binned.gaussian_ids_sorted, tile_bins, records, bg, img_h, img_w,
+                            block_x, block_y)
+            except BaseException:
+                S.drop_pending(binned)   # (out of memory, say)
+                raise
+            if process_fn is None:
+                gaussian_ids_sorted = binned.gaussian_ids_sorted
+                S._remember_capacity(hint_key, binned.num_intersects)
 
         ctx.save_for_backward(means2d, scales2d, rotation, colors, opacities, xys, depths, radii,
                               conics, gaussian_ids_sorted, tile_bins, final_Ts, final_idx, bg)

@@ -18,7 +18,7 @@ from typing import Optional
 import torch
 
 from . import _native as N
-from .splat import _dense, _give_pinned, _layout, _take_pinned
+from .splat import _dense, _give_pinned, _layout, _PendingCount, _take_pinned
 
 GS_RECORD_FLOATS = N.GS_RECORD_BYTES // 4
 
@@ -127,9 +127,9 @@ class GsBinned:
         self.num_intersects = 0
         self.grad_accum_clean = True
         # Set while the intersection count has not been read (bin_gaussians
-        # with a capacity hint): (pinned status buffer, capacity of the ids,
-        # cs_bin_finish into a new buffer); resolve_gaussians() settles it.
-        self.pending = None
+        # with a capacity hint); resolve_gaussians() settles it, drop_pending()
+        # gives it up.
+        self.pending: Optional[_PendingCount] = None
 
     def ptr(self, name: str) -> int:
         return self._base + self._table[name][0]
@@ -166,13 +166,13 @@ def resolve_gaussians(b: GsBinned) -> bool:
     size (outputs computed from the first build must be computed again)."""
     if b.pending is None:
         return False
-    pinned, capacity, finish = b.pending
+    pend = b.pending
     b.pending = None
-    I = b.num_intersects = _read_count(pinned)
-    if I <= capacity:
+    I = b.num_intersects = _read_count(pend.pinned)
+    if I <= pend.capacity:
         b.gaussian_ids_sorted = b.gaussian_ids_sorted[:I]
         return False
-    b.gaussian_ids_sorted = finish(I, None)
+    b.gaussian_ids_sorted = pend.finish(I)
     return True
 
 
@@ -211,7 +211,7 @@ def bin_gaussians(xys, conics, radii, depths, img_h: int, img_w: int, block_x: i
     status_host, event, status_dev = pinned[0], pinned[1], pinned[3]
     hip = N.hip()
 
-    def finish(capacity, status_out):
+    def finish(capacity, status_out=None):
         ids = torch.empty((capacity,), dtype=torch.int32, device=dev)
         with N.prof("gs.fwd.bin_finish"):
             N.call("cs_bin_finish", q_("order"), q_("rank_tile_ranges"), n, q_("status"),
@@ -224,13 +224,13 @@ def bin_gaussians(xys, conics, radii, depths, img_h: int, img_w: int, block_x: i
         capacity = max(1, int(capacity_hint))
         b.gaussian_ids_sorted = finish(capacity, status_dev)
         N.hip_check(hip.hipEventRecord(event, st), "hipEventRecord")
-        b.pending = (pinned, capacity, finish)
+        b.pending = _PendingCount(pinned, capacity, finish)
         return b
     N.hip_check(hip.hipMemcpyAsync(status_host.data_ptr(), q_("status"), 16,
                                    N.HIP_MEMCPY_DEVICE_TO_HOST, st), "hipMemcpyAsync")
     N.hip_check(hip.hipEventRecord(event, st), "hipEventRecord")
     I = b.num_intersects = _read_count(pinned)
-    b.gaussian_ids_sorted = finish(I, None)
+    b.gaussian_ids_sorted = finish(I)
     return b
 
 

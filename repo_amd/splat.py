@@ -480,8 +480,8 @@ def resolve_binned(b: Binned) -> bool:
     pend = b.pending
     if pend is None:
         return False
-    I = _read_count(pend, b.nseg)
     b.pending = None
+    I = _read_count(pend, b.nseg)
     b.num_intersects = I
     if I <= pend.capacity:
         b.primitive_ids_sorted = b.primitive_ids_sorted[:I]
@@ -490,6 +490,18 @@ def resolve_binned(b: Binned) -> bool:
     b.grad_accum_clean = True
     b.log_ctr_clean = True
     return True
+
+
+def drop_pending(b) -> None:
+    """Ends a binning whose intersection count nobody will read (its forward
+    raised): waits for the launch that writes the pinned status buffer, then
+    gives the buffer and its event back.  Nothing to do when it was read."""
+    pend = b.pending
+    if pend is None:
+        return
+    b.pending = None
+    N.hip_check(N.hip().hipEventSynchronize(pend.pinned[1]), "hipEventSynchronize")
+    _give_pinned(pend.pinned)
 
 
 def intersection_capacity(num_intersects: int) -> int:
@@ -1059,9 +1071,13 @@ def _splat_forward(ctx, mode, cubics_norm, primitive_seg_offsets, colors, opacit
     # requires a gradient).
     log = any(ctx.needs_input_grad)
     b.log_key = hint_key
-    out = _forward_launch(b, bg, log=log)
-    if resolve_binned(b):
+    try:
         out = _forward_launch(b, bg, log=log)
+        if resolve_binned(b):
+            out = _forward_launch(b, bg, log=log)
+    except BaseException:
+        drop_pending(b)   # (out of memory, say)
+        raise
     _remember_capacity(hint_key, b.num_intersects)
     if b.num_intersects <= 0:
         ctx.empty = True
