@@ -37,8 +37,10 @@ def project_cubics_2d_forward_tilelang(cubics_norm, stroke_widths, support_radii
     num_tiles_hit = torch.empty((n,), dtype=torch.int32, device=dev)
     if n == 0:
         return cubics_px, tile_ranges, num_tiles_hit
-    N.call("cs_project_cubics_2d_forward", N.ptr(_f32(cubics_norm)),
-           N.ptr(_f32(stroke_widths).view(-1)), N.ptr(_f32(support_radii).view(-1)), n,
+    # (Copies that a conversion makes are held until the launch: freed one by
+    # one they would all get the same memory.)
+    c, sw, sr = _f32(cubics_norm), _f32(stroke_widths).view(-1), _f32(support_radii).view(-1)
+    N.call("cs_project_cubics_2d_forward", N.ptr(c), N.ptr(sw), N.ptr(sr), n,
            int(img_height), int(img_width), int(block_x), int(block_y), float(aabb_pad),
            int(bool(aniso_intersects)), N.ptr(cubics_px), N.ptr(tile_ranges),
            N.ptr(num_tiles_hit), N.stream(dev))
@@ -68,10 +70,9 @@ def map_cubic_to_intersects_tilelang(tile_ranges, depths, cum_tiles_hit, tile_bo
                 torch.empty((0,), dtype=torch.int32, device=dev))
     isect_ids = torch.empty((num_intersects,), dtype=torch.int64, device=dev)
     curve_ids = torch.empty((num_intersects,), dtype=torch.int32, device=dev)
-    tr = _i32(tile_ranges)
-    N.call("cs_map_cubic_to_intersects", N.ptr(tr), N.ptr(_f32(depths).view(-1)),
-           N.ptr(_i32(cum_tiles_hit)), int(tr.shape[0]), int(tile_bounds[0]), N.ptr(isect_ids),
-           N.ptr(curve_ids), N.stream(dev))
+    tr, d, cum = _i32(tile_ranges), _f32(depths).view(-1), _i32(cum_tiles_hit)
+    N.call("cs_map_cubic_to_intersects", N.ptr(tr), N.ptr(d), N.ptr(cum), int(tr.shape[0]),
+           int(tile_bounds[0]), N.ptr(isect_ids), N.ptr(curve_ids), N.stream(dev))
     return isect_ids, curve_ids
 
 
@@ -199,6 +200,7 @@ def accumulate_edge_grads_to_cubics(v_edges, num_segments, *, distance_samples,
     if int(seo.numel()) != nseg + 1:
         raise ValueError(f"segment_edge_offsets size mismatch: got {int(seo.numel())}, "
                          f"expected {nseg + 1}")
-    N.call("cs_accumulate_edge_grads_csr", N.ptr(ve), N.ptr(_f32(edge_t_starts)),
-           N.ptr(_f32(edge_t_ends)), N.ptr(seo), nseg, 2, 2, N.ptr(v_px), None, N.stream(dev))
+    t0, t1 = _f32(edge_t_starts), _f32(edge_t_ends)
+    N.call("cs_accumulate_edge_grads_csr", N.ptr(ve), N.ptr(t0), N.ptr(t1), N.ptr(seo), nseg, 2,
+           2, N.ptr(v_px), None, N.stream(dev))
     return v_px

@@ -23,7 +23,9 @@ from .splat import _dense, _give_pinned, _layout, _PendingCount, _take_pinned
 GS_RECORD_FLOATS = N.GS_RECORD_BYTES // 4
 
 
-# (Only the tensors' addresses are taken.)
+# (Only the tensors' addresses are taken.  The results are held until the
+# launch: copies made by a conversion and freed one by one would all get the
+# same memory.)
 def _f32(t: torch.Tensor) -> torch.Tensor:
     return _dense(t, torch.float32)
 
@@ -80,11 +82,11 @@ def project_backward(scales2d, rotation, radii, conics, v_xy, v_conic, img_h: in
     v_rot = buf[4 * n:5 * n]
     v_cov = buf[5 * n:8 * n].view(n, 3) if with_cov2d else None
     meta = None if gaussian_meta is None else _i32(gaussian_meta).view(-1)
+    s, rad, q, vx, vq = _f32(scales2d), _i32(radii), _f32(conics), _f32(v_xy), _f32(v_conic)
     with N.prof("gs.bwd.proj"):
-        N.call("cs_gs_project_backward", N.ptr(_f32(scales2d)), N.ptr(r), N.ptr(_i32(radii)),
-               N.ptr(_f32(conics)), N.ptr(_f32(v_xy)), N.ptr(_f32(v_conic)), N.ptr(meta), n,
-               int(img_h), int(img_w), N.ptr(v_cov), N.ptr(v_mean), N.ptr(v_scale), N.ptr(v_rot),
-               N.stream(dev))
+        N.call("cs_gs_project_backward", N.ptr(s), N.ptr(r), N.ptr(rad), N.ptr(q), N.ptr(vx),
+               N.ptr(vq), N.ptr(meta), n, int(img_h), int(img_w), N.ptr(v_cov), N.ptr(v_mean),
+               N.ptr(v_scale), N.ptr(v_rot), N.stream(dev))
     return v_cov, v_mean, v_scale, v_rot
 
 
@@ -258,11 +260,11 @@ def rasterize_forward(gaussian_ids_sorted, tile_bins, records, background, img_h
     out = torch.empty((img_h, img_w, 3), dtype=torch.float32, device=dev)
     tid = torch.empty((2, img_h, img_w), dtype=torch.float32, device=dev)
     final_T, final_idx = tid[0], tid[1].view(torch.int32)
+    ids, bins, bg = _i32(gaussian_ids_sorted), _i32(tile_bins), _f32(background).view(-1)
     with N.prof("gs.fwd.rast"):
-        N.call("cs_gs_rasterize_forward", N.ptr(_i32(gaussian_ids_sorted)), N.ptr(_i32(tile_bins)),
-               N.ptr(records), N.ptr(_f32(background).view(-1)), int(img_h), int(img_w),
-               int(block_x), int(block_y), N.ptr(out), N.ptr(final_T), N.ptr(final_idx),
-               N.stream(dev))
+        N.call("cs_gs_rasterize_forward", N.ptr(ids), N.ptr(bins), N.ptr(records), N.ptr(bg),
+               int(img_h), int(img_w), int(block_x), int(block_y), N.ptr(out), N.ptr(final_T),
+               N.ptr(final_idx), N.stream(dev))
     return out, final_T, final_idx
 
 
@@ -283,13 +285,13 @@ def rasterize_backward(gaussian_ids_sorted, tile_bins, records, background, img_
     v_rgb, v_op = grads[5 * n:8 * n].view(n, 3), grads[8 * n:9 * n]
     meta = None if intersect_meta_sorted is None else _i32(intersect_meta_sorted).view(-1)
     va = None if v_output_alpha is None else _f32(v_output_alpha)
+    ids, bins, bg = _i32(gaussian_ids_sorted), _i32(tile_bins), _f32(background).view(-1)
+    fT, fi, vo = _f32(final_Ts), _i32(final_idx), _f32(v_output)
     with N.prof("gs.bwd.rast"):
-        N.call("cs_gs_rasterize_backward", N.ptr(_i32(gaussian_ids_sorted)), N.ptr(meta),
-               N.ptr(_i32(tile_bins)), N.ptr(records), N.ptr(_f32(background).view(-1)),
-               int(img_h), int(img_w), int(block_x), int(block_y), N.ptr(_f32(final_Ts)),
-               N.ptr(_i32(final_idx)), N.ptr(_f32(v_output)), N.ptr(va), N.ptr(v_xy),
-               N.ptr(v_conic), N.ptr(v_rgb), N.ptr(v_op), N.ptr(curve_contrib_rgb),
-               N.ptr(curve_isect_contrib), N.stream(dev))
+        N.call("cs_gs_rasterize_backward", N.ptr(ids), N.ptr(meta), N.ptr(bins), N.ptr(records),
+               N.ptr(bg), int(img_h), int(img_w), int(block_x), int(block_y), N.ptr(fT),
+               N.ptr(fi), N.ptr(vo), N.ptr(va), N.ptr(v_xy), N.ptr(v_conic), N.ptr(v_rgb),
+               N.ptr(v_op), N.ptr(curve_contrib_rgb), N.ptr(curve_isect_contrib), N.stream(dev))
     return v_xy, v_conic, v_rgb, v_op
 
 
@@ -309,9 +311,9 @@ def map_gaussian_to_intersects(num_points: int, num_intersects: int, xys, depths
         if conics.shape[0] != num_points:
             raise ValueError(
                 f"conics num_points mismatch: expected {num_points}, got {conics.shape[0]}")
-    N.call("cs_gs_map_to_intersects", N.ptr(_f32(xys)),
-           None if conics is None else N.ptr(_f32(conics)), N.ptr(_f32(depths).view(-1)),
-           N.ptr(_i32(radii).view(-1)), N.ptr(_i32(cum_tiles_hit).view(-1)), int(num_points),
-           int(num_intersects), int(tile_bounds_[0]), int(tile_bounds_[1]), int(block_x),
-           int(block_y), N.ptr(isect_ids), N.ptr(gaussian_ids), N.stream(dev))
+    xy, q, d = _f32(xys), None if conics is None else _f32(conics), _f32(depths).view(-1)
+    rad, cum = _i32(radii).view(-1), _i32(cum_tiles_hit).view(-1)
+    N.call("cs_gs_map_to_intersects", N.ptr(xy), N.ptr(q), N.ptr(d), N.ptr(rad), N.ptr(cum),
+           int(num_points), int(num_intersects), int(tile_bounds_[0]), int(tile_bounds_[1]),
+           int(block_x), int(block_y), N.ptr(isect_ids), N.ptr(gaussian_ids), N.stream(dev))
     return isect_ids, gaussian_ids

@@ -275,9 +275,9 @@ def rasterize_cubic_fill_backward_tilelang(tile_bounds, block, img_size, primiti
             if int(seo.numel()) != num_segments + 1:
                 raise ValueError(f"segment_edge_offsets size mismatch: got {int(seo.numel())}, "
                                  f"expected {num_segments + 1}")
-            N.call("cs_accumulate_edge_grads_csr", N.ptr(v_edges), N.ptr(_f32(edge_t_starts)),
-                   N.ptr(_f32(edge_t_ends)), N.ptr(seo), num_segments, H, W, N.ptr(v_px),
-                   N.ptr(v_norm), N.stream(dev))
+            t0, t1 = _f32(edge_t_starts), _f32(edge_t_ends)
+            N.call("cs_accumulate_edge_grads_csr", N.ptr(v_edges), N.ptr(t0), N.ptr(t1),
+                   N.ptr(seo), num_segments, H, W, N.ptr(v_px), N.ptr(v_norm), N.stream(dev))
         if v_px is not v_cubics_px:
             v_cubics_px.copy_(v_px)
         return v_cubics_px, v_colors, v_opacities, v_inv_sigma2s
@@ -296,8 +296,9 @@ def rasterize_cubic_fill_backward_tilelang(tile_bounds, block, img_size, primiti
             raise ValueError(f"segment_edge_offsets size mismatch: got {int(seo.numel())}, "
                              f"expected {num_segments + 1}")
         aux = torch.zeros((E, N.EDGE_AUX_INTS), dtype=torch.int32, device=dev)
-        N.call("cs_edge_aux_from_csr", N.ptr(seo), num_segments, N.ptr(_f32(edge_t_starts)),
-               N.ptr(_f32(edge_t_ends)), E, N.ptr(aux), N.stream(dev))
+        t0, t1 = _f32(edge_t_starts), _f32(edge_t_ends)
+        N.call("cs_edge_aux_from_csr", N.ptr(seo), num_segments, N.ptr(t0), N.ptr(t1), E,
+               N.ptr(aux), N.stream(dev))
         N.call("cs_rasterize_backward_de_casteljau", *common, N.ptr(aux), N.ptr(fT), N.ptr(fi),
                None, None, N.ptr(vo), 0, *grads)
     if v_px is not v_cubics_px:
