@@ -2894,8 +2894,8 @@ extern "C" int cs_rasterize_backward_counted(
                               stream);
 }
 
-extern "C" int32_t cs_raster_split_waves(int32_t nsub) {
-    return nsub > 0 ? split_waves(1, nsub) : 0;
+extern "C" int32_t cs_raster_split_waves(int32_t mode, int32_t nsub) {
+    return nsub > 0 && (mode == 0 || mode == 1) ? split_waves(mode, nsub) : 0;
 }
 
 extern "C" size_t cs_raster_tile_order_elems(int32_t ntiles) {

@@ -573,7 +573,7 @@ def _poll_log_use(key) -> None:
     _LOG_UNITS[key] = units
 
 
-def log_layout(key, capacity: int, nsub: int, waves_per_tile: int = 2):
+def log_layout(key, capacity: int, mode: int, nsub: int, waves_per_tile: int = 2):
     """(units per entry, pool bytes) for a forward of scene shape `key` with
     `capacity` list entries and tiles of `waves_per_tile` waves: the waves'
     own regions, plus shared blocks for a quarter of them and one block per
@@ -582,7 +582,7 @@ def log_layout(key, capacity: int, nsub: int, waves_per_tile: int = 2):
     _poll_log_use(key)
     units = _LOG_UNITS.get(key, LOG_FIRST_UNITS_PER_ENTRY)
     regions = 16 * waves_per_tile * capacity * units
-    waves = 2 * nsub * int(N.lib().cs_raster_split_waves(nsub))
+    waves = 2 * nsub * int(N.lib().cs_raster_split_waves(mode, nsub))
     shared = regions // 4 + waves * N.RASTER_LOG_BLOCK_BYTES + (1 << 20)
     return units, (16 + regions + shared + 255) // 256 * 256
 
@@ -676,7 +676,7 @@ def _forward_launch(b: Binned, background, eval_counts=None, log=True,
         key = b.log_key if b.log_key is not None else (
             dev.index, b.mode, b.nprim, b.nseg, H, W, b.samples, b.adaptive, b.block_x,
             b.block_y)
-        units, pool_bytes = log_layout(key, cap, nsub, wpt)
+        units, pool_bytes = log_layout(key, cap, b.mode, nsub, wpt)
         if log_pool_bytes_override is not None:
             units, pool_bytes = 0, max(16, int(log_pool_bytes_override) // 16 * 16)
         b.log_index = aux[2 * H * W:]
