@@ -901,11 +901,12 @@ __global__ __launch_bounds__(256) void k_split_half(const float* __restrict__ cu
 }
 
 // Depth ranks of at most kRankPairsMax keys: one launch of all-pairs
-// counting.  Up to kRankSortMax: the first stage ranks each block of
-// kRankBlock keys among themselves (k_prim_prep does it for the cubic path,
-// k_gs_keys_rects for the Gaussians, k_rank_blocks for the others), the second
-// merges the blocks (k_rank_merge).  Up to kRankSegmentsMax: the blocks are
-// merged into segments, and those into the order.  Above, the radix sort.
+// counting.  Up to kRankSegmentsMax, the launch that makes the keys
+// (k_prim_prep, k_gs_keys_rects) also ranks each block of kRankBlock keys
+// among themselves; up to kRankSortMax the blocks are merged in one launch
+// (k_rank_merge), above in two (k_rank_segments, k_rank_segment_merge).  Above
+// kRankSegmentsMax, the radix sort.  (cs_radix_sort_pairs_u32 takes the first
+// two ways too, with k_rank_blocks for the block ranks.)
 constexpr int kRankPairsMax = 8192;
 constexpr int kRankSortMax = 16384;
 constexpr int kRankBlock = 256;
@@ -2278,7 +2279,7 @@ extern "C" int cs_scan_exclusive_u32(const uint32_t* in, uint32_t* out, int32_t 
 extern "C" size_t cs_radix_counts_elems(int32_t n) {
     const int nb = blocks_for(n > 0 ? n : 1, kRsTile);
     const size_t radix = (size_t)256 * nb;
-    // The sort of at most kRankSortMax keys stages 2n words here.
+    // The sort of at most kRankSortMax keys stages 2n words here
     // (and so do the depth ranks of at most kRankSegmentsMax keys).
     const size_t rank = n > kRankPairsMax && n <= kRankSegmentsMax ? (size_t)2 * n : 0;
     return radix > rank ? radix : rank;
@@ -2346,8 +2347,9 @@ extern "C" int cs_radix_sort_pairs_u32(uint32_t* keys, int32_t* vals, uint32_t* 
 // smallest key (ties by primitive id) and rank_rects[r] its tile rectangle
 // (already written when `ranked`); per-tile counts, per-segment totals, then
 // the segments' first slots; status[0] receives the intersection total.
-static int rank_and_count(bool blocks_ranked, uint32_t* keys, int32_t* order,
-                          const int4* prim_rects,
+// kRankPairsMax < nprim <= kRankSegmentsMax: keys_alt and vals_alt hold the
+// blocks' sorted keys and ranks (from the launch that made the keys).
+static int rank_and_count(uint32_t* keys, int32_t* order, const int4* prim_rects,
                           int4* rank_rects, int nprim, int tbx, int tby, uint32_t* keys_alt,
                           int32_t* vals_alt, uint32_t* radix_counts, uint32_t* scan_temp,
                           uint32_t* tile_count,
@@ -2359,11 +2361,6 @@ static int rank_and_count(bool blocks_ranked, uint32_t* keys, int32_t* order,
                            keys, nprim, (const int32_t*)nullptr, (uint32_t*)nullptr,
                            (int32_t*)nullptr, prim_rects, order, rank_rects);
     } else if (nprim <= kRankSortMax) {
-        // Block ranks into keys_alt / vals_alt (already there when
-        // blocks_ranked: k_prim_prep wrote them).
-        if (!blocks_ranked)
-            hipLaunchKernelGGL(k_rank_blocks, dim3(blocks_for(nprim, kRankBlock)),
-                               dim3(kRankBlock), 0, stream, keys, nprim, keys_alt, vals_alt);
         hipLaunchKernelGGL(k_rank_merge<false>, dim3(blocks_for(nprim, kMergeKeys)),
                            dim3(kMergeThreads), 0, stream, keys,
                            keys_alt, vals_alt, nprim, (const int32_t*)nullptr,
@@ -2371,9 +2368,6 @@ static int rank_and_count(bool blocks_ranked, uint32_t* keys, int32_t* order,
     } else if (nprim <= kRankSegmentsMax) {
         // Segment keys and ids in radix_counts [2 nprim].
         int32_t* seg_ids = reinterpret_cast<int32_t*>(radix_counts + nprim);
-        if (!blocks_ranked)
-            hipLaunchKernelGGL(k_rank_blocks, dim3(blocks_for(nprim, kRankBlock)),
-                               dim3(kRankBlock), 0, stream, keys, nprim, keys_alt, vals_alt);
         hipLaunchKernelGGL(k_rank_segments, dim3(blocks_for(nprim, kWave)), dim3(kSegThreads), 0,
                            stream, keys, keys_alt, vals_alt, nprim, radix_counts, seg_ids);
         hipLaunchKernelGGL(k_rank_segment_merge, dim3(blocks_for(nprim, kWave)),
@@ -2521,7 +2515,7 @@ static int bin_prepare(const float* cubics_norm, const int32_t* seg_offsets, con
                            reinterpret_cast<int32_t*>(keys_alt),
                            reinterpret_cast<PrimRec*>(prim_recs), order,
                            reinterpret_cast<int4*>(rank_tile_ranges));
-        return rank_and_count(true, keys, order, reinterpret_cast<const int4*>(prim_tile_ranges),
+        return rank_and_count(keys, order, reinterpret_cast<const int4*>(prim_tile_ranges),
                               reinterpret_cast<int4*>(rank_tile_ranges), nprim, tbx, tby,
                               keys_alt, vals_alt, radix_counts, scan_temp, tile_count,
                               tile_scratch, status, stream, true);
@@ -2535,7 +2529,7 @@ static int bin_prepare(const float* cubics_norm, const int32_t* seg_offsets, con
                        reinterpret_cast<PrimRec*>(prim_recs),
                        nprim <= kRankSegmentsMax ? keys_alt : nullptr,
                        nprim <= kRankSegmentsMax ? vals_alt : nullptr);
-    return rank_and_count(true, keys, order, reinterpret_cast<const int4*>(prim_tile_ranges),
+    return rank_and_count(keys, order, reinterpret_cast<const int4*>(prim_tile_ranges),
                           reinterpret_cast<int4*>(rank_tile_ranges), nprim, tbx, tby, keys_alt,
                           vals_alt, radix_counts, scan_temp, tile_count,
                           tile_scratch, status, stream);
@@ -2706,7 +2700,7 @@ extern "C" int cs_gs_bin_prepare(const float* xys, const float* conics, const in
                        conics, radii, depths, n, block_x, block_y, tbx, tby,
                        reinterpret_cast<int4*>(tile_rects), keys, order, status,
                        blocks ? keys_alt : nullptr, blocks ? vals_alt : nullptr);
-    return rank_and_count(blocks, keys, order, reinterpret_cast<const int4*>(tile_rects),
+    return rank_and_count(keys, order, reinterpret_cast<const int4*>(tile_rects),
                           reinterpret_cast<int4*>(rank_tile_ranges), n, tbx, tby, keys_alt,
                           vals_alt, radix_counts, scan_temp, tile_count,
                           tile_scratch, status, stream);
