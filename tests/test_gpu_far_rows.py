@@ -12,13 +12,16 @@ import torch
 
 from helpers import check_grads, hip_bin, oracle_forward, random_v_out
 from oracle import oracle as O
+from repo_amd import _native as N
 from repo_amd import splat, synth
 
-H, W = 150, 190
+# Canvases of launches with eight waves on a 16 x 8 block, with four and with
+# one (120, 600 and 1332 sub-blocks); the scenes grow with them.
+CANVASES = {8: (150, 190), 4: (371, 393), 1: (561, 577)}
 
 
-def _drifted(seed, drift, nseg, S, P=24):
-    sc = synth.small_scene(seed, P=P, nseg=nseg, h=H, w=W, S=S, rmin=4.0, rmax=70.0)
+def _drifted(seed, drift, nseg, S, H, W, P=24):
+    sc = synth.small_scene(seed, P=P, nseg=nseg, h=H, w=W, S=S, rmin=4.0, rmax=0.47 * H)
     g = torch.Generator("cpu").manual_seed(seed + 77)
     half = torch.tensor([W / 2.0, H / 2.0])
     sc.cubics_norm = sc.cubics_norm + drift * torch.randn(sc.cubics_norm.shape, generator=g) / half
@@ -26,12 +29,12 @@ def _drifted(seed, drift, nseg, S, P=24):
     return sc
 
 
-def _spiral(turns, S=4):
+def _spiral(turns, H, W, S=4):
     """One chain of `turns` loops around the image centre (4 cubics a loop,
     shrinking), ending away from its start, above a drifted scene."""
-    sc = _drifted(5, 0.02, 4, S, P=6)
+    sc = _drifted(5, 0.02, 4, S, H, W, P=6)
     k = torch.arange(4 * turns + 1, dtype=torch.float32)
-    th, r = k * (math.pi / 2), 60.0 - 10.0 * k / k[-1]
+    th, r = k * (math.pi / 2), 0.4 * H - 10.0 * k / k[-1]
     p = torch.stack([W / 2 + r * th.cos(), H / 2 + r * th.sin()], 1)
     t = torch.stack([-th.sin(), th.cos()], 1) * (r * 0.5523).unsqueeze(1)
     cub = torch.stack([p[:-1], p[:-1] + t[:-1], p[1:] - t[1:], p[1:]], 1)
@@ -50,12 +53,12 @@ def _spiral(turns, S=4):
 
 
 SCENES = {
-    "tiny_gaps": lambda: _drifted(0, 0.02, 4, 16),
-    "pixel_gaps": lambda: _drifted(1, 1.5, 4, 16),
-    "exactly_64_edges": lambda: _drifted(2, 0.3, 4, 17),
-    "two_chunks": lambda: _drifted(3, 0.3, 3, 24),
-    "four_chunks": lambda: _drifted(4, 0.3, 9, 24),
-    "winding_beyond_a_byte": lambda: _spiral(150),
+    "tiny_gaps": lambda h, w: _drifted(0, 0.02, 4, 16, h, w),
+    "pixel_gaps": lambda h, w: _drifted(1, 1.5, 4, 16, h, w),
+    "exactly_64_edges": lambda h, w: _drifted(2, 0.3, 4, 17, h, w),
+    "two_chunks": lambda h, w: _drifted(3, 0.3, 3, 24, h, w),
+    "four_chunks": lambda h, w: _drifted(4, 0.3, 9, 24, h, w),
+    "winding_beyond_a_byte": lambda h, w: _spiral(150, h, w),
 }
 
 
@@ -65,10 +68,13 @@ def _bits(a):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", list(SCENES))
-@pytest.mark.parametrize("counted", [False, True])
-def test_far_edges_count_per_row(name, counted):
-    sc = SCENES[name]()
-    print(f"[far rows] {name} counted={counted}", flush=True)
+@pytest.mark.parametrize("waves,counted", [(8, False), (8, True), (4, False), (1, False)])
+def test_far_edges_count_per_row(name, waves, counted):
+    """(The counting instances always take one wave.)"""
+    h, w = CANVASES[waves]
+    assert N.lib().cs_raster_split_waves(splat.MODE_FILL, splat.sub_blocks(h, w)) == waves
+    sc = SCENES[name](h, w)
+    print(f"[far rows] {name} waves={waves} counted={counted}", flush=True)
     b, s = hip_bin(sc)
     bg = s.background.float().contiguous()
     counts = torch.zeros(5, dtype=torch.int64, device="cuda") if counted else None

@@ -17,6 +17,10 @@ structured cases hold one at a time meet here. The properties are:
 * sample counts S from 2 to 33;
 * tile lists longer than 64 entries (every fourth scene).
 
+The 48 scenes' images are at most 329 x 329 pixels, where the raster puts eight
+waves on each 16 x 8 block.  Some of the scenes are drawn again on canvases of
+the sizes that take four waves and one, there with the adaptive flattening too.
+
 Bars: the image, T and index are bit-exact. The gradients are within
 1e-4 |ref| + 1e-6 max|ref| per element (the order of the fp32 sums differs
 from the oracle's float64 ones).
@@ -25,18 +29,23 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import check_grads, hip_bin, oracle_forward, random_v_out, scene_np
+from helpers import (check_grads, grad_scale_tol, hip_bin, oracle_forward, random_v_out,
+                     scene_np)
 from oracle import oracle as O
+from repo_amd import _native as N
 from repo_amd import splat, synth
 
 SEEDS = list(range(48))
 
 
-def _fuzz_scene(seed):
+def _fuzz_scene(seed, canvas=None):
+    """Scene `seed`, on a canvas (h, w) of its own size unless one is given."""
     rng = np.random.default_rng(9000 + seed)
     big = seed % 4 == 3        # lists longer than one 64-entry chunk
     h = int(rng.integers(100, 330) if big else rng.integers(17, 140))
     w = int(rng.integers(100, 330) if big else rng.integers(17, 170))
+    if canvas is not None:
+        h, w = canvas
     P = int(rng.integers(100, 260) if big else rng.integers(1, 48))
     stroke = seed % 3 == 2
     S = int(rng.choice([2, 3, 7, 8, 16, 33]))
@@ -107,12 +116,15 @@ def _bits(a):
 @pytest.mark.gpu
 @pytest.mark.parametrize("seed", SEEDS)
 def test_random_scene_forward_bit_exact_and_backward(seed):
-    sc = _fuzz_scene(seed)
+    _check_scene(seed, _fuzz_scene(seed))
+
+
+def _check_scene(seed, sc, flatten="bernstein"):
     print(f"[fuzz] seed {seed}: {sc.img_h}x{sc.img_w}, P={sc.num_primitives}, S={sc.S}, "
           f"stroke={sc.stroke_widths is not None}", flush=True)
-    b, s = hip_bin(sc)
+    b, s = hip_bin(sc, flatten_method=flatten)
     out, T, idx = splat.rasterize_forward(b, s.background.float().contiguous())
-    fw = oracle_forward(sc)
+    fw = oracle_forward(sc, flatten_method=flatten)
     np.testing.assert_array_equal(_bits(out.cpu().numpy()), _bits(fw["out"]))
     np.testing.assert_array_equal(_bits(T.cpu().numpy()), _bits(fw["final_T"]))
     np.testing.assert_array_equal(idx.cpu().numpy(), fw["final_idx"])
@@ -127,7 +139,33 @@ def test_random_scene_forward_bit_exact_and_backward(seed):
               ("v_aa_widths", v_aa, g["v_aa_widths"])]
     if v_sw is not None:
         checks.append(("v_stroke_widths", v_sw, g["v_stroke_widths"]))
-    check_grads(checks)
+    if flatten == "bernstein":
+        check_grads(checks)
+    else:   # (the bar of the adaptive flattening's own tests)
+        for name, got, ref in checks:
+            ok, err = grad_scale_tol(got.cpu().numpy(), ref)
+            assert ok, (name, err)
+
+
+# (waves per 16 x 8 block, mode) -> canvas of that launch: 600, 1332 and 2450
+# sub-blocks.
+CANVASES = {(4, splat.MODE_FILL): (371, 393), (4, splat.MODE_STROKE): (371, 393),
+            (1, splat.MODE_FILL): (561, 577), (1, splat.MODE_STROKE): (777, 793)}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("waves", [4, 1])
+@pytest.mark.parametrize("seed,flatten", [(s, "bernstein") for s in range(16)]
+                         + [(s, "de_casteljau") for s in (3, 5, 7, 8, 10, 11)])
+def test_random_scene_on_a_canvas_of_fewer_waves(seed, flatten, waves):
+    """Forward (with the log) and backward of the launches that larger images
+    take; the counting instances, which always take one wave, are other code."""
+    mode = splat.MODE_STROKE if seed % 3 == 2 else splat.MODE_FILL
+    h, w = CANVASES[waves, mode]
+    assert N.lib().cs_raster_split_waves(mode, splat.sub_blocks(h, w)) == waves
+    sc = _fuzz_scene(seed, (h, w))
+    assert (sc.stroke_widths is not None) == (mode == splat.MODE_STROKE)
+    _check_scene(seed, sc, flatten)
 
 
 BLOCKS = [(16, 16), (8, 8), (16, 8), (32, 16), (24, 24), (48, 32)]
