@@ -7,9 +7,10 @@ current stream; there is no CPU or torch fallback.  The binning replaces the
 reference's cumsum + map + torch.sort + tile-bin pass
 (tilelang_renderer.py:224-269) with depth ranks and per-tile counting lists
 (cs_gs_bin_prepare / cs_bin_finish), which produce the same
-gaussian_ids_sorted and tile_bins; one host read of the intersection count
-sizes gaussian_ids_sorted (the reference reads the same count,
-tilelang_renderer.py:54-58).
+gaussian_ids_sorted and tile_bins.  The host reads the intersection count once
+a forward (the reference reads the same count, tilelang_renderer.py:54-58): to
+size gaussian_ids_sorted, or, given a capacity from an earlier forward, after
+the raster is enqueued, to trim the buffer or to build the lists again.
 """
 from __future__ import annotations
 

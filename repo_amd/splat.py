@@ -652,7 +652,7 @@ def forward_state(b: Binned):
 # Launches over at most this many sub-blocks take no tile order: all of their
 # workgroups are resident at once (512 blocks of eight waves, two or more per
 # CU), so it does not matter in which order they start.
-ORDER_MIN_SUB_BLOCKS = 256
+UNORDERED_SUB_BLOCKS = 256
 
 
 def _forward_launch(b: Binned, background, eval_counts=None, log=True,
@@ -700,7 +700,7 @@ def _forward_launch(b: Binned, background, eval_counts=None, log=True,
     # The tile order is kept apart: the next forward reads it after this
     # forward's buffers are gone.
     okey = (dev.index, st, nsub)
-    if nsub <= ORDER_MIN_SUB_BLOCKS and eval_counts is None:
+    if nsub <= UNORDERED_SUB_BLOCKS and eval_counts is None:
         prev, age, remake = None, 0, False
     else:
         prev = _TILE_ORDERS.get(okey)
