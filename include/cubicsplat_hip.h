@@ -244,12 +244,13 @@ int cs_bin_finish(const int32_t* order, const int32_t* rank_tile_ranges, int32_t
  * over the XCDs in turn (balance for skewed scenes). */
 size_t cs_raster_tile_order_elems(int32_t ntiles);
 
-/* Waves per 16 x 8 pixel block of a raster launch over nsub 16 x 16 sub-blocks
- * (1, or more for small images; mode as in cs_bin_prepare; 0 for nsub <= 0 or
- * another mode; no reference counterpart).  Each of them may reserve a block of
- * CS_RASTER_LOG_BLOCK_BYTES of the raster log's pool past the per-wave
- * regions. */
-int32_t cs_raster_split_waves(int32_t mode, int32_t nsub);
+/* Waves per 16 x 8 pixel block of a forward (backward != 0: a backward) raster
+ * launch over nsub 16 x 16 sub-blocks (1, or more for small images; mode as in
+ * cs_bin_prepare; 0 for nsub <= 0 or another mode; no reference counterpart).
+ * Each wave of a forward may reserve a block of CS_RASTER_LOG_BLOCK_BYTES of
+ * the raster log's pool past the per-wave regions.  A log serves a backward of
+ * any wave count. */
+int32_t cs_raster_split_waves(int32_t mode, int32_t nsub, int32_t backward);
 int cs_raster_tile_order(const uint32_t* wave_cost, int32_t ntiles, int32_t chunked,
                          int32_t* tile_order, hipStream_t stream);
 

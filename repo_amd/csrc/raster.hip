@@ -487,7 +487,7 @@ __device__ __forceinline__ SubBlock sub_block(const TileGrid& tg,
 // an entry and pixel, the same operations in the same order as one wave would
 // run, so the results are bit-identical), so no state is handed back.
 // Training step of 64 paths at 128 x 128: forward 135 -> 41 us, backward
-// 73 -> 24 us; the rule is at split_waves.
+// 73 -> 24 us; the rules are at split_waves_fwd.
 __device__ __forceinline__ SubBlock split_block(const TileGrid& tg,
                                                 const int32_t* __restrict__ tile_order) {
     if (tile_order) {
@@ -504,19 +504,31 @@ __device__ __forceinline__ SubBlock split_block(const TileGrid& tg,
 // Waves per block of a launch over nsb sub-blocks (1: not split).  A launch
 // that leaves the chip idle takes as long as its longest list; splitting
 // shortens that, but every wave repeats the cull tests and the recurrence,
-// which costs more than it saves once the launch fills the chip.  Measured
-// (us, one, 4 and 8 waves; fills at one path per 400 pixels, strokes at one
-// per 67), forward and backward:
+// which costs more than it saves once the launch fills the chip.  The backward
+// has more of both (its reductions and gradient buffer are per wave) and gives
+// way earlier.  Measured (us, rocprofv3; one, 4 and 8 waves; square images;
+// fills of one path per 400 pixels, strokes of one path of three cubics per
+// 150):
 //   sub-blocks    fill forward     fill backward    stroke forward   stroke backward
-//        64     46 / 28 / 19     33 / 27 / 25     54 / 28 / 20     65 / 40 / 34
-//       475     64 / 44 / 40     47 / 33 / 37     74 / 39 / 35     84 / 47 / 50
-//      1024     71 / 64 / 71     58 / 51 / 64     78 / 53 / 55     89 / 62 / 76
-//      1536     76 / 79 / 96     59 / 61 / 83     84 / 65 / 74     96 / 76 / 98
-//      2565     80 / 103 / 140   67 / 81 / 114    93 / 91 / 113    105 / 102 / 145
-// (16 waves are no faster at 64 and slower from 256 on; two waves gain
-// little at 950 and nothing at 1536.)
-__host__ __forceinline__ int split_waves(int mode, int nsb) {
-    return nsb <= 512 ? 8 : nsb <= (mode == 0 ? 1152 : 2304) ? 4 : 1;
+//        64     59 / 35 / 29     18 / 11 /  9     65 / 31 / 21     31 / 16 / 12
+//       256     70 / 45 / 34     26 / 16 / 13     68 / 39 / 29     33 / 17 / 15
+//       484     82 / 56 / 44     32 / 18 / 23     69 / 39 / 39     36 / 19 / 25
+//      1024     75 / 61 / 71     38 / 33 / 45     78 / 55 / 59     37 / 30 / 42
+//      1156     89 / 66 / 73     36 / 35 / 51     87 / 59 / 65     43 / 31 / 44
+//      1444     89 / 70 / 89     43 / 42 / 63     83 / 65 / 78     40 / 39 / 57
+//      1600     84 / 74 / 98     39 / 47 / 71     81 / 70 / 83     40 / 41 / 59
+//      2025     81 / 85 / 120    42 / 54 / 84     92 / 89 / 105    49 / 52 / 79
+//      2209     76 / 86 / 120    43 / 60 / 92     87 / 92 / 112    50 / 54 / 84
+// The limits hold for sparser, denser and longer paths too: at each, none of
+// them is slower than with one wave.  (Fills of 186 edges, backward: 30 / 27 /
+// 40 at 1024, 27 / 28 / 40 at 1156, which is why the fills' backward ends at
+// 1024.  An image with four paths in all loses 0.5 us of 8.5 in the forward
+// from 484 on.)
+__host__ __forceinline__ int split_waves_fwd(int mode, int nsb) {
+    return nsb <= 512 ? 8 : nsb <= (mode == 0 ? 1152 : 2048) ? 4 : 1;
+}
+__host__ __forceinline__ int split_waves_bwd(int mode, int nsb) {
+    return nsb <= 256 ? 8 : nsb <= (mode == 0 ? 1024 : 1408) ? 4 : 1;
 }
 
 // One entry of a split round, left in LDS for the block's waves: its alpha at
@@ -2538,7 +2550,7 @@ static void launch_fwd(const RasterArgs& a) {
     const FwdTail tail{a.bg,        a.out,    a.out_planes, a.final_T, a.final_idx,
                        a.wave_cost, a.counts, a.out_planar, a.img_h,   a.img_w};
     if constexpr (!COUNT) {
-        switch (split_waves(MODE, a.tg.nsb)) {
+        switch (split_waves_fwd(MODE, a.tg.nsb)) {
             case 8: return launch_fwd_split<MODE, 8>(a, tail);
             case 4: return launch_fwd_split<MODE, 4>(a, tail);
             default: break;
@@ -2569,7 +2581,7 @@ static void launch_bwd5(const RasterArgs& a) {
 
 template <int MODE, bool COUNT, bool ADAPTIVE, bool LEAN>
 static void launch_bwd4(const RasterArgs& a) {
-    switch (COUNT ? 1 : split_waves(MODE, a.tg.nsb)) {
+    switch (COUNT ? 1 : split_waves_bwd(MODE, a.tg.nsb)) {
         case 8: launch_bwd5<MODE, COUNT, ADAPTIVE, LEAN, COUNT ? 1 : 8>(a); break;
         case 4: launch_bwd5<MODE, COUNT, ADAPTIVE, LEAN, COUNT ? 1 : 4>(a); break;
         default: launch_bwd5<MODE, COUNT, ADAPTIVE, LEAN, 1>(a); break;
@@ -2894,8 +2906,9 @@ extern "C" int cs_rasterize_backward_counted(
                               stream);
 }
 
-extern "C" int32_t cs_raster_split_waves(int32_t mode, int32_t nsub) {
-    return nsub > 0 && (mode == 0 || mode == 1) ? split_waves(mode, nsub) : 0;
+extern "C" int32_t cs_raster_split_waves(int32_t mode, int32_t nsub, int32_t backward) {
+    if (nsub <= 0 || (mode != 0 && mode != 1)) return 0;
+    return backward ? split_waves_bwd(mode, nsub) : split_waves_fwd(mode, nsub);
 }
 
 extern "C" size_t cs_raster_tile_order_elems(int32_t ntiles) {

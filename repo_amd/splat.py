@@ -582,7 +582,7 @@ def log_layout(key, capacity: int, mode: int, nsub: int, waves_per_tile: int = 2
     _poll_log_use(key)
     units = _LOG_UNITS.get(key, LOG_FIRST_UNITS_PER_ENTRY)
     regions = 16 * waves_per_tile * capacity * units
-    waves = 2 * nsub * int(N.lib().cs_raster_split_waves(mode, nsub))
+    waves = 2 * nsub * int(N.lib().cs_raster_split_waves(mode, nsub, 0))
     shared = regions // 4 + waves * N.RASTER_LOG_BLOCK_BYTES + (1 << 20)
     return units, (16 + regions + shared + 255) // 256 * 256
 

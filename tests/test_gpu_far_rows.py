@@ -72,7 +72,9 @@ def _bits(a):
 def test_far_edges_count_per_row(name, waves, counted):
     """(The counting instances always take one wave.)"""
     h, w = CANVASES[waves]
-    assert N.lib().cs_raster_split_waves(splat.MODE_FILL, splat.sub_blocks(h, w)) == waves
+    for backward in (0, 1):
+        assert N.lib().cs_raster_split_waves(splat.MODE_FILL, splat.sub_blocks(h, w),
+                                             backward) == waves
     sc = SCENES[name](h, w)
     print(f"[far rows] {name} waves={waves} counted={counted}", flush=True)
     b, s = hip_bin(sc)

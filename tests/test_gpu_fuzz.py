@@ -147,8 +147,8 @@ def _check_scene(seed, sc, flatten="bernstein"):
             assert ok, (name, err)
 
 
-# (waves per 16 x 8 block, mode) -> canvas of that launch: 600, 1332 and 2450
-# sub-blocks.
+# (waves per 16 x 8 block, mode) -> canvas whose two launches take that many:
+# 600, 1332 and 2450 sub-blocks.
 CANVASES = {(4, splat.MODE_FILL): (371, 393), (4, splat.MODE_STROKE): (371, 393),
             (1, splat.MODE_FILL): (561, 577), (1, splat.MODE_STROKE): (777, 793)}
 
@@ -162,7 +162,8 @@ def test_random_scene_on_a_canvas_of_fewer_waves(seed, flatten, waves):
     take; the counting instances, which always take one wave, are other code."""
     mode = splat.MODE_STROKE if seed % 3 == 2 else splat.MODE_FILL
     h, w = CANVASES[waves, mode]
-    assert N.lib().cs_raster_split_waves(mode, splat.sub_blocks(h, w)) == waves
+    for backward in (0, 1):
+        assert N.lib().cs_raster_split_waves(mode, splat.sub_blocks(h, w), backward) == waves
     sc = _fuzz_scene(seed, (h, w))
     assert (sc.stroke_widths is not None) == (mode == splat.MODE_STROKE)
     _check_scene(seed, sc, flatten)

@@ -13,18 +13,20 @@ from repo_amd import _native as N
 from repo_amd import splat, synth
 
 
-def _waves(mode, nsub):
-    return int(N.lib().cs_raster_split_waves(mode, nsub))
+def _waves(mode, nsub, backward=0):
+    return int(N.lib().cs_raster_split_waves(mode, nsub, backward))
 
 
 @pytest.mark.parametrize("mode", [splat.MODE_FILL, splat.MODE_STROKE])
-def test_the_wave_count_falls_with_the_image(mode):
-    assert _waves(mode, 0) == 0 and _waves(2, 5) == 0 and _waves(mode, 1) == 8
-    assert all(_waves(mode, n) >= _waves(mode, n + 1) for n in range(1, 4000))
-    assert _waves(mode, 1 << 20) == 1
+@pytest.mark.parametrize("backward", [0, 1])
+def test_the_wave_count_falls_with_the_image(mode, backward):
+    assert _waves(mode, 0, backward) == 0 and _waves(2, 5, backward) == 0
+    counts = [_waves(mode, n, backward) for n in range(1, 4000)]
+    assert counts[0] == 8 and counts == sorted(counts, reverse=True)
+    assert _waves(mode, 1 << 20, backward) == 1
 
 
-@pytest.mark.parametrize("mode,last", [(splat.MODE_FILL, 1152), (splat.MODE_STROKE, 2304)])
+@pytest.mark.parametrize("mode,last", [(splat.MODE_FILL, 1152), (splat.MODE_STROKE, 2048)])
 def test_log_pool_holds_a_block_for_each_wave_of_the_launch(mode, last):
     """The pool's size follows the launch's own wave count: past the last size
     that is split, one wave per 16 x 8 block."""
@@ -36,7 +38,8 @@ def test_log_pool_holds_a_block_for_each_wave_of_the_launch(mode, last):
         assert 0 <= size - (16 + regions + regions // 4 + blocks + (1 << 20)) < 256
 
 
-# name: (H, W, paths, stroke); sub-blocks 1, 512, 513, 1152 | 1153, 2304 | 2305.
+# name: (H, W, paths, stroke), by the sub-blocks where a wave count changes
+# (forward 512, 1152 and 2048, backward 256, 1024 and 1408) and just past them.
 SIZES = {
     "one_block": (9, 13, 150, False),
     "ragged": (75, 100, 300, False),
@@ -44,8 +47,20 @@ SIZES = {
     "fill_513": (144, 912, 60, False),
     "fill_1152": (384, 768, 60, False),
     "stroke_ragged": (75, 100, 400, True),
-    "stroke_2304": (768, 768, 80, True),
+    "stroke_2048": (512, 1024, 80, True),
+    "fill_256": (256, 256, 60, False),
+    "fill_260": (208, 320, 60, False),
+    "fill_1024": (512, 512, 80, False),
+    "fill_1025": (400, 656, 80, False),
+    "stroke_256": (256, 256, 60, True),
+    "stroke_260": (208, 320, 60, True),
+    "stroke_1408": (512, 704, 90, True),
+    "stroke_1410": (480, 752, 90, True),
 }
+FORWARD = ("one_block", "ragged", "fill_512", "fill_513", "fill_1152", "stroke_ragged",
+           "stroke_2048")
+BACKWARD = ("one_block", "ragged", "stroke_ragged", "fill_513", "fill_256", "fill_260",
+            "fill_1024", "fill_1025", "stroke_256", "stroke_260", "stroke_1408", "stroke_1410")
 
 
 def _scene(name):
@@ -59,7 +74,7 @@ def _bits(a):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name", list(SIZES))
+@pytest.mark.parametrize("name", FORWARD)
 @pytest.mark.parametrize("flatten", ["bernstein", "de_casteljau"])
 def test_split_equals_one_wave(name, flatten):
     sc = _scene(name)
@@ -77,7 +92,7 @@ def test_split_equals_one_wave(name, flatten):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name", ["one_block", "ragged", "stroke_ragged", "fill_513"])
+@pytest.mark.parametrize("name", BACKWARD)
 @pytest.mark.parametrize("pool", [None, 1 << 14])
 def test_split_backward(name, pool):
     """Gradients and contribution outputs, with a full log and with one whose
