@@ -605,8 +605,8 @@ __global__ __launch_bounds__(kWave * kFlattenWaves) void k_project_flatten_wave(
     }
 }
 
-// Adaptive flattening for at most kDecasLaneDepth halvings, both passes with a
-// group of L = max(2, 2^maxd) lanes per segment instead of a thread (a thread
+// Adaptive flattening for at most kDecasLaneDepth halvings and
+// decas_lane_segments segments, both passes with a group of L = max(2, 2^maxd) lanes per segment instead of a thread (a thread
 // walks up to 2^maxd leaves from the root one after the other).  Bound by the
 // latency of the descent (a root and a division a level) and of the owner
 // search.  8192 segments, S = 24: counting 61 -> 8.8 us, writing 62 -> 11.3 us,
@@ -616,6 +616,22 @@ __global__ __launch_bounds__(kWave * kFlattenWaves) void k_project_flatten_wave(
 // holds the finest interval i; the leaf is the first such lane's.  The segments
 // are projected and staged as in k_project_flatten_wave.
 constexpr int kDecasLaneDepth = 6;
+// A group always takes its L lanes, a thread only the leaves that there are, so
+// with enough segments to fill the chip by threads the groups lose, first where
+// the segments are flat.  The limit is where they do not even there (records
+// and lists included, us, threads against groups; flat segments of 3 to 6
+// pixels, and rings of up to 120):
+//   segments, S     flat        rings           segments, S     flat        rings
+//   131072,  3     53 / 52     54 / 52         262144,  3     68 / 72     69 / 73
+//   131072,  5     59 / 56     67 / 58         262144,  5     76 / 80     94 / 81
+//    65536,  9     54 / 48     70 / 50         131072,  9     60 / 64     91 / 67
+//    32768, 17     53 / 44    112 / 49          65536, 17     54 / 55    122 / 63
+//    32768, 24     52 / 51    135 / 60          40000, 24     57 / 67    136 / 78
+//    16384, 65     54 / 45    132 / 54          40000, 65     57 / 87    136 / 107
+// (The figures at S = 33 and 49 are those at 24 and 65: what counts is L.)
+constexpr int decas_lane_segments(int maxd) {
+    return maxd <= 2 ? 1 << 17 : maxd <= 4 ? (1 << 19) >> maxd : (1 << 20) >> maxd;
+}
 // Segments per workgroup (as flatten_segs; the descent is the longer part).
 __host__ __device__ constexpr int decas_segs(int lanes) { return lanes >= 32 ? 16 : 32; }
 
@@ -701,7 +717,9 @@ __global__ __launch_bounds__(kWave * kFlattenWaves) void k_decas_project(
 // `offsets` null the workgroup makes its segments' edge offsets itself, from
 // the counts of all earlier segments, and writes them to seg_edge_offsets
 // (one launch and its single-workgroup scan less; the caller does so up to
-// kDecasOwnScan segments, where reading the counts costs no more).
+// kDecasOwnScan segments, where reading the counts costs no more: all binning
+// launches with the scan and without, S = 9, 32.4 / 25.5 us at 8192 segments,
+// 41.9 / 30.0 at 16384, 39.1 / 36.7 at 24576, 42.8 / 41.9 at 32768).
 constexpr int kDecasOwnScan = 32768;
 
 template <int L>
@@ -2423,7 +2441,8 @@ static int bin_prepare(const float* cubics_norm, const int32_t* seg_offsets, con
         return CS_ERR_ARGS;
     }
     const int tbx = (img_w + block_x - 1) / block_x, tby = (img_h + block_y - 1) / block_y;
-    const bool lane_decas = adaptive && nseg > 0 && maxd <= kDecasLaneDepth;
+    const bool lane_decas = adaptive && nseg > 0 && maxd <= kDecasLaneDepth &&
+                            nseg <= decas_lane_segments(maxd);
     if (!adaptive && nseg > 0 && samples <= kWave) {
         // One lane per sample point; the kernel also sets the status words.
         const int lanes = samples <= 2 ? 2 : 1 << ceil_log2(samples);

@@ -1,7 +1,7 @@
 """Adaptive flattening with a group of lanes per segment: every depth the lane
 groups take (S = 2 ... 65) and the first the per-thread walk takes (66),
 degenerate and far segments, a last workgroup that is not full, and more
-segments than a workgroup sums the counts of.  Edges, CSR and aux records bit
+segments than a workgroup sums the counts of or than the groups are taken for.  Edges, CSR and aux records bit
 for bit against the oracle, and cull and segment records against the per-vertex
 ones."""
 import numpy as np
@@ -59,9 +59,12 @@ def test_every_depth(S):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("P", [1, 10923, 10924])
-def test_segment_counts(P):
-    """3, 32769 (the scan's first) and 32772 segments."""
-    print(f"[decas lanes] P={P}", flush=True)
-    sc = synth.small_scene(4, P=P, nseg=3, h=64, w=64, S=6, rmax=12.0)
+@pytest.mark.parametrize("P,S", [(1, 6), (10923, 6), (10924, 6), (43690, 3), (43691, 3),
+                                 (10922, 24), (10923, 24), (5461, 65), (5462, 65)])
+def test_segment_counts(P, S):
+    """3, 32769 (the scan's first) and 32772 segments; the last counts that take
+    lane groups and the first that do not: 131070 and 131073 segments at S = 3,
+    32766 and 32769 at 24, 16383 and 16386 at 65."""
+    print(f"[decas lanes] P={P} S={S}", flush=True)
+    sc = synth.small_scene(4, P=P, nseg=3, h=64, w=64, S=S, rmax=12.0)
     _check(sc)
