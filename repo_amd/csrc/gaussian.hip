@@ -559,14 +559,26 @@ static inline int gs_wg(int32_t block_x, int32_t block_y, int kp) {
     return (block_x * block_y + per_wave - 1) / per_wave * kWave;
 }
 
-// Two pixels per lane where that halves the waves and leaves four for each of
-// the chip's 1024 SIMDs; with fewer, a launch lasts as long as its longest
-// list, and one pixel per lane shortens each entry.  Measured, one against two
-// (us, forward + backward): 8192 waves of two (1024 x 1024) 137 + 395 against
-// 131 + 294, 620 (317 x 241) 22 + 48 against 33 + 59.
-static inline bool gs_two_pixels(int32_t block_x, int32_t block_y, int ntiles) {
+// Two pixels per lane where that halves the waves and leaves at least
+// `min_waves`; with fewer, a launch lasts as long as its longest list, and one
+// pixel per lane shortens each entry.  The forward needs six waves for each of
+// the chip's 1024 SIMDs, the backward, which has more to share between two
+// pixels, two.  Measured, one against two (us; 16 x 8 tiles, a Gaussian of up to
+// 8 pixels per 10 pixels | of up to 20 per 100):
+//   waves of two     forward                    backward
+//       1536     54 /  68 | 30 / 34         114 / 113 |  84 /  70
+//       2048     60 /  71 | 30 / 33         129 / 118 |  83 /  67
+//       4096     83 /  97 | 44 / 43         227 / 156 | 132 /  90
+//       5120    102 / 107 | 48 / 49         292 / 174 | 147 / 103
+//       6144    116 / 120 | 54 / 54         339 / 211 | 171 / 116
+//       8192    147 / 145 | 64 / 64         402 / 260 | 185 / 124
+// (16 x 16 tiles: the forward 101 / 111 at 5120 and 116 / 114 at 6144, the
+// backward 105 / 116 at 1536 and 127 / 121 at 2048.)
+constexpr int kGsTwoForward = 6144, kGsTwoBackward = 2048;
+
+static inline bool gs_two_pixels(int32_t block_x, int32_t block_y, int ntiles, int min_waves) {
     const int two = gs_wg(block_x, block_y, 2);
-    return gs_wg(block_x, block_y, 1) == 2 * two && (int64_t)ntiles * (two / kWave) >= 4096;
+    return gs_wg(block_x, block_y, 1) == 2 * two && (int64_t)ntiles * (two / kWave) >= min_waves;
 }
 
 extern "C" int cs_gs_rasterize_forward(const int32_t* gaussian_ids_sorted,
@@ -578,7 +590,7 @@ extern "C" int cs_gs_rasterize_forward(const int32_t* gaussian_ids_sorted,
     if (!gs_dims_ok(img_h, img_w, block_x, block_y) || !al(records, 16)) return CS_ERR_ARGS;
     const int tbx = (img_w + block_x - 1) / block_x, tby = (img_h + block_y - 1) / block_y;
     const int ntiles = tbx * tby;
-    const bool two = gs_two_pixels(block_x, block_y, ntiles);
+    const bool two = gs_two_pixels(block_x, block_y, ntiles, kGsTwoForward);
     hipLaunchKernelGGL(two ? k_gs_raster_fwd<2> : k_gs_raster_fwd<1>, dim3(ntiles),
                        dim3(gs_wg(block_x, block_y, two ? 2 : 1)), 0, stream,
                        gaussian_ids_sorted, tile_bins, reinterpret_cast<const GsRec*>(records),
@@ -597,7 +609,7 @@ extern "C" int cs_gs_rasterize_backward(
     if (!gs_dims_ok(img_h, img_w, block_x, block_y) || !al(records, 16)) return CS_ERR_ARGS;
     const int tbx = (img_w + block_x - 1) / block_x, tby = (img_h + block_y - 1) / block_y;
     const int ntiles = tbx * tby;
-    const bool two = gs_two_pixels(block_x, block_y, ntiles);
+    const bool two = gs_two_pixels(block_x, block_y, ntiles, kGsTwoBackward);
     const int threads = gs_wg(block_x, block_y, two ? 2 : 1);
     auto kern = contrib_rgb || isect_contrib
                     ? (two ? k_gs_raster_bwd<2, true> : k_gs_raster_bwd<1, true>)

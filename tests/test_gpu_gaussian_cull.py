@@ -10,14 +10,15 @@ import torch
 from helpers import grad_scale_tol
 from oracle import oracle as O
 
-# name: (n, H, W, block_x, block_y); two pixels per lane from 4096 waves of
-# 128 pixels on.
+# name: (n, H, W, block_x, block_y); two pixels per lane from 6144 waves of 128
+# pixels on in the forward and 2048 in the backward (6240, 2080 and 8694 here).
 CASES = {
     "one_pixel_16x8": (600, 120, 150, 16, 8),
     "odd_block_5x7": (300, 60, 70, 5, 7),
     "wide_block_128x2": (300, 50, 260, 128, 2),
     "one_wave_of_64": (300, 64, 96, 8, 8),
-    "two_pixels_16x8": (400, 512, 1030, 16, 8),
+    "two_pixels_16x8": (400, 768, 1030, 16, 8),
+    "two_pixels_backward_16x8": (400, 256, 1030, 16, 8),
     "two_pixels_24x16": (400, 736, 1500, 24, 16),
 }
 
