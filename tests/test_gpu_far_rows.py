@@ -1,7 +1,7 @@
 """Filled chains with gaps between their segments, as an optimizer leaves them
 (each segment's copy of a shared end point moves by itself): the raster sums
 the crossings of the edges right of a wave per pixel row from their cull words.
-Chains of fewer and more than 64 edges, gaps below and above a pixel, long
+Chains of fewer and more than 64, 256 and 384 edges, gaps below and above a pixel, long
 spirals (winding numbers beyond a byte) and both fill rules, bit for bit
 against the oracle, and the gradients."""
 import math
@@ -58,6 +58,11 @@ SCENES = {
     "exactly_64_edges": lambda h, w: _drifted(2, 0.3, 4, 17, h, w),
     "two_chunks": lambda h, w: _drifted(3, 0.3, 3, 24, h, w),
     "four_chunks": lambda h, w: _drifted(4, 0.3, 9, 24, h, w),
+    "six_chunks": lambda h, w: _drifted(6, 0.3, 15, 24, h, w),
+    "closed_three_chunks": lambda h, w: _drifted(7, 0.0, 7, 24, h, w),
+    "256_edges": lambda h, w: _drifted(8, 0.05, 16, 17, h, w),
+    "closed_384_edges": lambda h, w: _drifted(9, 0.0, 24, 17, h, w),
+    "closed_seven_chunks": lambda h, w: _drifted(10, 0.0, 17, 24, h, w),
     "winding_beyond_a_byte": lambda h, w: _spiral(150, h, w),
 }
 
