@@ -1428,7 +1428,10 @@ __global__ __launch_bounds__(kMergeThreads) void k_rank_merge(
 // search steps.  The four-pass radix sort that larger counts take runs 256
 // keys at a time per workgroup and is bound by its three barriers a step:
 // 24576 keys 98 -> 19 us, 100000 keys 109 -> 26 us (with the rectangles'
-// gather; and 4 us more in the launch that ranks the blocks).
+// gather; and 4 us more in the launch that ranks the blocks).  The searches
+// grow with the square of the count; at the limit, all binning launches before
+// the lists take 201 -> 175 us for 262144 Gaussians and 220 -> 195 for strokes
+// (152 -> 79 and 164 -> 91 at 131072).
 constexpr int kSegmentKeys = 4096;
 constexpr int kSegMergeWaves = 4;
 constexpr int kSegThreads = kWave * kSegMergeWaves;

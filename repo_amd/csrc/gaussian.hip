@@ -183,7 +183,7 @@ __device__ __forceinline__ float gs_exp(float sigma, bool mid) {
 // whose ellipse misses the wave's pixels.  KP = 2 halves the scalar work and
 // the record loads per pixel and is taken when that still fills the chip
 // (gs_two_pixels).  100000 Gaussians at 1024 x 1024, 16 x 8 tiles: 171 -> 132
-// us, all of it issue time of its vector instructions (SQ_INSTS_VALU).
+// us, all of it issue time of its vector instructions (VALU busy 99%).
 template <int KP>
 __global__ __launch_bounds__(1024 / KP) void k_gs_raster_fwd(
     const int32_t* __restrict__ ids, const int32_t* __restrict__ bins_g,

@@ -487,7 +487,7 @@ __device__ __forceinline__ SubBlock sub_block(const TileGrid& tg,
 // an entry and pixel, the same operations in the same order as one wave would
 // run, so the results are bit-identical), so no state is handed back.
 // Training step of 64 paths at 128 x 128: forward 135 -> 41 us, backward
-// 73 -> 24 us; the rules are at split_waves_fwd.
+// 73 -> 26 us; the rules are at split_waves_fwd.
 __device__ __forceinline__ SubBlock split_block(const TileGrid& tg,
                                                 const int32_t* __restrict__ tile_order) {
     if (tile_order) {
