@@ -3,9 +3,8 @@
 One step = render (fused binning + forward raster) of 4096 closed cubic paths
 (4 segments, S=16) at 2040x1356 -> clamp(0,1) -> NCHW -> loss
 MSE + 0.2 * (1 - SSIM(11, 1.5)) against the synthetic target -> backward ->
-Adam on control points and colors.  Prints one JSON line (see the contract
-in the repository's build notes).  --config N runs BASELINE.json's config N
-instead (1-5, each with its own loss; see WORKLOADS).
+Adam on control points and colors.  Prints one JSON line.  --config N runs
+workload N instead (1-5, each with its own loss; see WORKLOADS).
 
 python bench.py [--gpus 1] [--steps 100] [--warmup 10] [--config 3] [--no-cpu-baseline]
 """
@@ -90,7 +89,7 @@ def render(sc, cub, col):
         sc.background, aa_widths=sc.aa_widths, distance_samples=sc.S)
 
 
-# The configurations of BASELINE.json: workload text and SSIM weight of the
+# The five workloads: workload text and SSIM weight of the
 # loss (0: MSE only).
 WORKLOADS = {
     1: ("64 closed cubic paths x 4 segments, S=8, 128x128, MSE", 0.0),
