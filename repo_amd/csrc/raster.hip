@@ -519,11 +519,13 @@ __device__ __forceinline__ SubBlock split_block(const TileGrid& tg,
 //      1600     84 / 74 / 98     39 / 47 / 71     81 / 70 / 83     40 / 41 / 59
 //      2025     81 / 85 / 120    42 / 54 / 84     92 / 89 / 105    49 / 52 / 79
 //      2209     76 / 86 / 120    43 / 60 / 92     87 / 92 / 112    50 / 54 / 84
-// The limits hold for sparser, denser and longer paths too: at each, none of
-// them is slower than with one wave.  (Fills of 186 edges, backward: 30 / 27 /
+// The limits hold for denser and longer paths too: at each, none of them is
+// slower than with one wave.  (Fills of 186 edges, backward: 30 / 27 /
 // 40 at 1024, 27 / 28 / 40 at 1156, which is why the fills' backward ends at
-// 1024.  An image with four paths in all loses 0.5 us of 8.5 in the forward
-// from 484 on.)
+// 1024.  The exception is a nearly empty image: with four paths in all, 484 to
+// 1024 sub-blocks lose 0.3 to 1.5 us of 9 in the forward and 1 to 2.5 of 9 in
+// the backward, whose pass the host bounds by far.  Adaptive flattening and
+// contribution outputs follow the same figures.)
 __host__ __forceinline__ int split_waves_fwd(int mode, int nsb) {
     return nsb <= 512 ? 8 : nsb <= (mode == 0 ? 1152 : 2048) ? 4 : 1;
 }
